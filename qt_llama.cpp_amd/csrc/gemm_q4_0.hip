@@ -43,6 +43,9 @@
 //     per row) and their f16 scales are loaded with coalesced loads into
 //     registers one chunk ahead, turned into signed bytes once (both K
 //     halves) and staged through kNBuf LDS buffers, one barrier per chunk.
+//
+// Products of few tokens, which would leave most SIMDs without a wave, run
+// as gemm_q4_0_few_kernel instead (K split over waves, below).
 
 #include <mutex>
 
@@ -400,6 +403,237 @@ __global__ __launch_bounds__(64 * kGemmWaves) void gemm_q4_0_mfma_kernel(const G
     }
 }
 
+// ---- few tokens ----------------------------------------------------------------
+// A handful of tokens (a chat turn, the tail of a prompt) gives the tile
+// kernel above few waves, each alone on its SIMD with the whole K loop in
+// front of it: 2304 x 9216 at 12 tokens was 72 waves of 288 blocks and took
+// 58 us for 12 MB of weights.  Only the block-ordered adds are serial; the
+// block terms are not.  So here a workgroup owns 16 rows x 16 tokens, P
+// producer waves split K four blocks at a time and write finished terms to
+// LDS, and four adder waves, one lane per output, add them in block order:
+//   round r: producer p forms blocks 4(rP + p)..+3 (one 16x16x32 MFMA each),
+//            the adders add round r-1; one barrier a round, two term buffers.
+// GLU: the gate and up products of the same rows in one workgroup (adder
+// lanes run both chains) and act = gelu_tanh(g) * u written directly, so the
+// two products never go through memory.
+//
+// A CU's vector memory path looks at adjacent lanes together, so every load
+// has adjacent lanes on adjacent bytes, and the operands are turned into the
+// MFMA's lane order (lane l: row or token l%16, K slots of quarter l/16) in
+// registers or in a private kilobyte of LDS:
+//   weights: lane 4r + b loads block b of row r (64 contiguous bytes a row);
+//     through LDS lane (row, quarter p) gets block p, then a 4x4 dword
+//     transpose over the quarters (four v_permlane swaps) hands quarter q dword q
+//     of all four blocks: values 4q..4q+3 (low nibbles) and 16+4q..+3 (high);
+//   tokens: quarter 2b + h loads half h of block b (two loads for four
+//     blocks), and the same transpose gives quarter q dword q of both halves;
+//   token scales: lane 16q + 4b + e loads token 4q + e of block b, which the
+//     scale products read as a row broadcast (a DPP operand, no instruction).
+constexpr int kFewRows = 16, kFewTokens = 16;
+constexpr int kFewAdders = 4;  // waves; kFewRows * kFewTokens lanes
+
+// Quarter q of a: dword q of block j for j = 0..3, from quarter p holding dwords 0..3 of block p.
+__device__ __forceinline__ void quarter_transpose(u32x4 &a)
+{
+    const auto s02 = __builtin_amdgcn_permlane32_swap(a.x, a.z, false, false);
+    const auto s13 = __builtin_amdgcn_permlane32_swap(a.y, a.w, false, false);
+    const auto lo = __builtin_amdgcn_permlane16_swap(s02[0], s13[0], false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(s02[1], s13[1], false, false);
+    a = u32x4{lo[0], lo[1], hi[0], hi[1]};
+}
+
+// Lane N of each 16-lane row, in every lane of the row.
+template <int N>
+__device__ __forceinline__ float row_bcast(float v)
+{
+    return __builtin_bit_cast(float,
+                              __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x150 + N, 0xf, 0xf, true));
+}
+
+// Terms of block J (of the wave's four) for tokens 4q..4q+3 and the lane's row.
+template <int J>
+__device__ __forceinline__ void few_terms(uint32_t w, uint32_t x0, uint32_t x1, float dw, float da, float (&t)[4][4])
+{
+    const v4i cm = {kMagicBits, kMagicBits, kMagicBits, kMagicBits};
+    const uint64_t bw = (uint64_t)(uint32_t)sbytes(w, 0) | ((uint64_t)(uint32_t)sbytes(w, 4) << 32);
+    const uint64_t ax = (uint64_t)x0 | ((uint64_t)x1 << 32);
+    const v4i d = __builtin_amdgcn_mfma_i32_16x16x32_i8((long)ax, (long)bw, cm, 0, 0, 0);
+    const int d0 = d[0], d1 = d[1], d2 = d[2], d3 = d[3];
+    t[0][J] = (__builtin_bit_cast(float, d0) - kMagic) * (row_bcast<4 * J>(da) * dw);
+    t[1][J] = (__builtin_bit_cast(float, d1) - kMagic) * (row_bcast<4 * J + 1>(da) * dw);
+    t[2][J] = (__builtin_bit_cast(float, d2) - kMagic) * (row_bcast<4 * J + 2>(da) * dw);
+    t[3][J] = (__builtin_bit_cast(float, d3) - kMagic) * (row_bcast<4 * J + 3>(da) * dw);
+}
+
+template <bool GLU, int P>
+__global__ __launch_bounds__(64 * (kFewAdders + P), GLU ? 4 : 6) void gemm_q4_0_few_kernel(const GemmMats mats,
+                                                                                 const uint8_t *__restrict__ gp,
+                                                                                 float *__restrict__ y, int rows,
+                                                                                 int nb, int batch, int ngroups,
+                                                                                 int ldy)
+{
+    constexpr int NM = GLU ? 2 : 1;              // products of the workgroup's rows
+    constexpr int NOUT = kFewRows * kFewTokens;  // outputs of each
+    constexpr int RB = 4 * P;                    // blocks a round
+    __shared__ __align__(16) float4 terms[2][NM][P][NOUT];  // [..][producer][token*16 + row] its 4 blocks
+    __shared__ __align__(16) u32x4 wq[P][NM][64];           // a producer's weights: row*4 + (block ^ row/4)
+    __shared__ __align__(16) float wd[P][NM][64];           // and their scales: row*4 + block
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int nrt = (rows + kFewRows - 1) / kFewRows;
+    const int rt = blockIdx.x % nrt, ts = blockIdx.x / nrt;  // row tile, token tile
+    const int r0 = rt * kFewRows;
+    const int rounds = (nb + RB - 1) / RB;
+
+    if (wave < kFewAdders) {
+        const int o = tid;
+        float acc[NM];
+#pragma unroll
+        for (int m = 0; m < NM; ++m) acc[m] = 0.0f;
+        for (int r = 0; r < rounds; ++r) {
+            lds_barrier();
+            float4 t[NM][P];
+#pragma unroll
+            for (int p = 0; p < P; ++p)
+#pragma unroll
+                for (int m = 0; m < NM; ++m) t[m][p] = terms[r & 1][m][p][o];
+            const int left = nb - r * RB;  // blocks of this round that exist
+            if (left >= RB) {
+#pragma unroll
+                for (int p = 0; p < P; ++p)
+#pragma unroll
+                    for (int m = 0; m < NM; ++m) {
+                        acc[m] = acc[m] + t[m][p].x;
+                        acc[m] = acc[m] + t[m][p].y;
+                        acc[m] = acc[m] + t[m][p].z;
+                        acc[m] = acc[m] + t[m][p].w;
+                    }
+            } else {
+#pragma unroll
+                for (int p = 0; p < P; ++p)
+#pragma unroll
+                    for (int m = 0; m < NM; ++m) {
+                        if (4 * p + 0 < left) acc[m] = acc[m] + t[m][p].x;
+                        if (4 * p + 1 < left) acc[m] = acc[m] + t[m][p].y;
+                        if (4 * p + 2 < left) acc[m] = acc[m] + t[m][p].z;
+                        if (4 * p + 3 < left) acc[m] = acc[m] + t[m][p].w;
+                    }
+            }
+        }
+        const int tok = ts * kFewTokens + (o >> 4), row = r0 + (o & 15);
+        if (tok < batch && row < rows) {
+            float *at = y + (size_t)tok * ldy + row;
+            if constexpr (GLU) *at = gelu_tanh(acc[0]) * acc[NM - 1];
+            else *at = acc[0];
+        }
+        return;
+    }
+
+    // Producer.  GLU: product m is matrix m, both of `rows` rows; otherwise
+    // the rows are stacked and the tile belongs to one matrix.
+    int mi = 0, mbase = 0;
+    if constexpr (!GLU)
+        while (mi + 1 < mats.n && r0 >= mbase + mats.rows[mi]) mbase += mats.rows[mi++];
+    const uint32_t mrows = (uint32_t)mats.rows[mi], qs_bytes = mrows * nb * 16;
+    __amdgpu_buffer_rsrc_t wr[NM];
+#pragma unroll
+    for (int m = 0; m < NM; ++m)
+        wr[m] = __builtin_amdgcn_make_buffer_rsrc((void *)mats.w[mi + m], (short)0,
+                                                  (int)(qs_bytes + mrows * nb * 2), kBufferFlags);
+    const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)gp, (short)0, (int)((uint32_t)ngroups * nb * 1152), kBufferFlags);
+    const int p = wave - kFewAdders, l16 = lane & 15, q = lane >> 4;
+    const int g = ts >> 1, t0 = kFewTokens * (ts & 1);  // token group, first token in it
+    // the lane's offsets in round 0
+    const uint32_t blk = (uint32_t)(r0 - mbase + (lane >> 2)) * nb + 4 * p + (lane & 3);
+    const uint32_t w_off = blk * 16, s_off = qs_bytes + blk * 2;
+    const uint32_t x_off = (((uint32_t)g * nb + 4 * p + (q >> 1)) * 64 + 32 * (q & 1) + t0 + l16) * 16;
+    const uint32_t d_off = (uint32_t)ngroups * nb * 1024 +
+                           (((uint32_t)g * nb + 4 * p + (l16 >> 2)) * 32 + t0 + 4 * q + (l16 & 3)) * 4;
+    const int w_put = (lane & ~3) + ((lane & 3) ^ ((lane >> 4) & 3)), w_get = 4 * l16 + (q ^ (l16 >> 2));
+
+    // Loads of a round past the last one are pointed past the buffer (they
+    // return zeros without touching memory); blocks past a row's last read
+    // whatever follows and are never added.
+    constexpr uint32_t kPast = 0xFFFF0000u;
+    struct WLoad {
+        u32x4 w[NM];
+        uint32_t s[NM];
+    };
+    struct XLoad {
+        u32x4 x[2];  // blocks 0, 1 and 2, 3
+        float da;
+    };
+    auto load_w = [&](int r, WLoad &o) {
+        const uint32_t wo = r < rounds ? w_off + (uint32_t)r * (RB * 16) : kPast;
+        const uint32_t so = r < rounds ? s_off + (uint32_t)r * (RB * 2) : kPast;
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            o.w[m] = __builtin_amdgcn_raw_buffer_load_b128(wr[m], wo, 0, 0);
+            o.s[m] = __builtin_amdgcn_raw_buffer_load_b16(wr[m], so, 0, 0);
+        }
+    };
+    auto load_x = [&](int r, XLoad &o) {
+        const uint32_t xo = r < rounds ? x_off + (uint32_t)r * (RB * 1024) : kPast;
+        const uint32_t dq = r < rounds ? d_off + (uint32_t)r * (RB * 128) : kPast;
+        o.x[0] = __builtin_amdgcn_raw_buffer_load_b128(gr, xo, 0, 0);
+        o.x[1] = __builtin_amdgcn_raw_buffer_load_b128(gr, xo + 2048, 0, 0);
+        o.da = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(gr, dq, 0, 0));
+    };
+    // A round's weights in the MFMA's lane order (LDS is in order within the wave).
+    u32x4 w[NM];
+    float4 dw[NM];
+    auto turn_w = [&](const WLoad &l) {
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            wq[p][m][w_put] = l.w[m];
+            wd[p][m][lane] = f16_bits_to_f32(l.s[m]);
+        }
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            w[m] = wq[p][m][w_get];
+            dw[m] = *reinterpret_cast<const float4 *>(&wd[p][m][4 * l16]);
+        }
+    };
+    auto round = [&](int r, WLoad &wl, WLoad &wn, XLoad &xl) {
+        quarter_transpose(xl.x[0]);
+        quarter_transpose(xl.x[1]);
+        float t[NM][4][4];  // [product][token 4q + e][block]
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            quarter_transpose(w[m]);
+            few_terms<0>(w[m].x, xl.x[0].x, xl.x[0].y, dw[m].x, xl.da, t[m]);
+            few_terms<1>(w[m].y, xl.x[0].z, xl.x[0].w, dw[m].y, xl.da, t[m]);
+            few_terms<2>(w[m].z, xl.x[1].x, xl.x[1].y, dw[m].z, xl.da, t[m]);
+            few_terms<3>(w[m].w, xl.x[1].z, xl.x[1].w, dw[m].w, xl.da, t[m]);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // (or the scheduler gathers the loads and waits for all of them)
+        load_w(r + 2, wl);
+        load_x(r + 2, xl);
+        __builtin_amdgcn_sched_barrier(0);
+        turn_w(wn);
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                terms[r & 1][m][p][(4 * q + e) * 16 + l16] =
+                    make_float4(t[m][e][0], t[m][e][1], t[m][e][2], t[m][e][3]);
+        lds_barrier();
+    };
+    WLoad wl[2];
+    XLoad xl[2];
+    load_w(0, wl[0]);  // in the order the rounds issue them (loads return in order)
+    load_x(0, xl[0]);
+    load_w(1, wl[1]);
+    load_x(1, xl[1]);
+    turn_w(wl[0]);
+    for (int r = 0;;) {
+        round(r, wl[0], wl[1], xl[0]);
+        if (++r == rounds) break;
+        round(r, wl[1], wl[0], xl[1]);
+        if (++r == rounds) break;
+    }
+}
+
 // Device scratch of the allocation-free GEMM entry point
 // (mrml_hip_gemm_q4_0_noalloc): the GEMM pack of its activations lives in
 // this file-scope array, one copy per GPU, held until the process ends.  Host
@@ -475,6 +709,46 @@ int launch_gemm_pack_from_act(mrml_hip_ctx *ctx, const void *pack, void *gpack, 
     return check_launch(ctx, "gemm_pack_from_act_kernel");
 }
 
+static int few_workgroups(int32_t rows, int32_t batch)
+{
+    return (rows + kFewRows - 1) / kFewRows * ((batch + kFewTokens - 1) / kFewTokens);
+}
+
+// Whether a product runs as gemm_q4_0_few_kernel.  A workgroup costs about
+// 8.5e-5 us a block there once the chip is full; the tile kernel takes 0.2 us
+// a block for anything up to one wave a SIMD (a lone wave's step), so the
+// line is at 0.2 / 8.5e-5 workgroups.  Measured on both sides of it:
+// 9216 x 2304 at 64 tokens (2304 workgroups) 17.6 against 19.7 us, at 80
+// (2880) 21.4 against 20.0; 4096 x 2304 at 128 (2048) 15.5 against 18.1;
+// 2304 x 9216 at 128 (1152) 28.4 against 58.7.
+bool gemm_few(int32_t rows, int32_t batch)
+{
+    return (int64_t)(rows + kFewRows - 1) / kFewRows * ((batch + kFewTokens - 1) / kFewTokens) <= 2304;
+}
+
+// Producers: 8 while the workgroups leave CUs their LDS (two of them a CU),
+// else 4 (up to four a CU).  2304 x 9216 at 16 tokens (144 workgroups) 9.6
+// with 8, 12.6 us with 4; at 48 (432) 13.8 and 15.0; 4096 x 2304 at 24 (512)
+// 7.1 and 6.4.  GLU holds two products' terms, so it takes 4: 9216 x 2304 at
+// 12 tokens 16.2 us, 21.0 with 8 (two tile products and the elementwise pass:
+// 42.5).
+static int launch_gemm_few(mrml_hip_ctx *ctx, bool glu, const GemmMats &mats, const void *gpack, float *y,
+                           int32_t rows, int nb, int32_t batch, int32_t ldy)
+{
+    const int ng = gemm_groups(batch), wgs = few_workgroups(rows, batch);
+    const dim3 grid((unsigned)wgs);
+    if (glu)
+        hipLaunchKernelGGL((gemm_q4_0_few_kernel<true, 4>), grid, dim3(64 * (kFewAdders + 4)), 0, ctx->stream, mats,
+                           (const uint8_t *)gpack, y, rows, nb, batch, ng, ldy);
+    else if (wgs < 448)
+        hipLaunchKernelGGL((gemm_q4_0_few_kernel<false, 8>), grid, dim3(64 * (kFewAdders + 8)), 0, ctx->stream, mats,
+                           (const uint8_t *)gpack, y, rows, nb, batch, ng, ldy);
+    else
+        hipLaunchKernelGGL((gemm_q4_0_few_kernel<false, 4>), grid, dim3(64 * (kFewAdders + 4)), 0, ctx->stream, mats,
+                           (const uint8_t *)gpack, y, rows, nb, batch, ng, ldy);
+    return check_launch(ctx, "gemm_q4_0_few_kernel");
+}
+
 static int launch_gemm_mats(mrml_hip_ctx *ctx, const GemmMats &mats, const void *gpack, float *y, int32_t rows,
                             int32_t cols, int32_t batch, int32_t ldy, bool relaxed)
 {
@@ -483,6 +757,7 @@ static int launch_gemm_mats(mrml_hip_ctx *ctx, const GemmMats &mats, const void 
     if (ldy < rows || ((uintptr_t)y & 3) != 0)
         return fail(ctx, MRML_HIP_E_INVALID, "gemm_q4_0: output stride %d below rows %d, or y not 4-byte aligned",
                     ldy, rows);
+    if (!relaxed && gemm_few(rows, batch)) return launch_gemm_few(ctx, false, mats, gpack, y, rows, nb, batch, ldy);
     const int vec = (ldy % 4 == 0 && ((uintptr_t)y & 15) == 0) ? 1 : 0;  // float4 stores reach every output row
     // FULL waves, one per (row tile, token group).  When they number just
     // over one per SIMD (down at M = 512: 1152 for 1024), the SIMDs holding
@@ -513,6 +788,24 @@ int launch_gemm_q4_0(mrml_hip_ctx *ctx, const void *w, const void *gpack, float 
     mats.rows[0] = rows;
     mats.n = 1;
     return launch_gemm_mats(ctx, mats, gpack, y, rows, cols, batch, ldy, relaxed);
+}
+
+// act = gelu_tanh(Wg x) * (Wu x) of every token over one GEMM pack, gu: 2*batch*rows floats
+int launch_gemm_q4_0_geglu(mrml_hip_ctx *ctx, const void *wg, const void *wu, const void *gpack, float *act, float *gu,
+                           int32_t rows, int32_t cols, int32_t batch)
+{
+    if (gemm_few(rows, batch)) {
+        GemmMats mats{};
+        mats.w[0] = (const uint8_t *)wg;
+        mats.w[1] = (const uint8_t *)wu;
+        mats.rows[0] = mats.rows[1] = rows;
+        mats.n = 2;
+        return launch_gemm_few(ctx, true, mats, gpack, act, rows, cols / 32, batch, rows);
+    }
+    const size_t n = (size_t)batch * rows;
+    if (int rc = launch_gemm_q4_0(ctx, wg, gpack, gu, rows, cols, batch)) return rc;
+    if (int rc = launch_gemm_q4_0(ctx, wu, gpack, gu + n, rows, cols, batch)) return rc;
+    return launch_geglu_rows(ctx, gu, gu + n, act, (int)n);
 }
 
 // Up to three products over one GEMM pack in one launch, their outputs

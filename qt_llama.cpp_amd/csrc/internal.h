@@ -112,6 +112,12 @@ int launch_gemm_q4_0(mrml_hip_ctx *ctx, const void *w, const void *gpack, float 
                      int32_t batch, int32_t ldy = 0, bool relaxed = false);
 int launch_gemm_q4_0_stacked(mrml_hip_ctx *ctx, const void *const *w, const int32_t *rows, int n, const void *gpack,
                              float *y, int32_t cols, int32_t batch, int32_t ldy, bool relaxed = false);
+// Whether an exact product of this size takes the few-token kernel (a relaxed one never does: the tile
+// kernel's one-FMA fold is slower there than the few-token kernel's exact one).
+bool gemm_few(int32_t rows, int32_t batch);
+// act = gelu_tanh(Wg x) * (Wu x) of every token ([batch][rows], unpadded rows); gu: 2*batch*rows floats of scratch
+int launch_gemm_q4_0_geglu(mrml_hip_ctx *ctx, const void *wg, const void *wu, const void *gpack, float *act, float *gu,
+                           int32_t rows, int32_t cols, int32_t batch);
 
 // Argmax whose final pass can also advance a device-side decode loop
 // (state = {token, pos}) and record the processed token in the recent-token

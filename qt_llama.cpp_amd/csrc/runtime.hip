@@ -700,11 +700,9 @@ int mrml_hip_gemm_q4_0_geglu(mrml_hip_ctx *ctx, const void *wg, const void *wu, 
     const size_t pk = align_up(gemm_pack_bytes(cols, batch), 256), n = (size_t)batch * rows;
     uint8_t *ws = (uint8_t *)workspace(ctx, pk + 2 * n * sizeof(float));
     if (!ws) return MRML_HIP_E_ALLOC;
-    float *g = reinterpret_cast<float *>(ws + pk), *u = g + n;
+    float *g = reinterpret_cast<float *>(ws + pk);
     if (int rc = launch_gemm_pack_quantize(ctx, x, ws, cols, batch)) return rc;
-    if (int rc = launch_gemm_q4_0(ctx, wg, ws, g, rows, cols, batch)) return rc;
-    if (int rc = launch_gemm_q4_0(ctx, wu, ws, u, rows, cols, batch)) return rc;
-    return launch_geglu_rows(ctx, g, u, act, (int)n);
+    return launch_gemm_q4_0_geglu(ctx, wg, wu, ws, act, g, rows, cols, batch);
 }
 
 size_t mrml_hip_gemm_pack_bytes(int32_t cols, int32_t batch)

@@ -169,6 +169,37 @@ def test_gemm_q4_0_split_tiles_bit_exact(backend, dev, orc, synth, rows, cols, b
     assert_bit_exact(run_gemm(backend, dev, w, x, rows, cols, batch, prequantised=True), ref, "pack entry")
 
 
+# Few tokens (16 rows x 16 tokens a workgroup, rounds of 32 or 16 blocks): one
+# block, partial and whole last rounds of an odd and even number, ragged row
+# and token tiles, both producer counts (448 workgroups and more take the
+# smaller), and the two sides of the line to the tile kernel (2304
+# workgroups), the tile kernel's with a K tail.
+@pytest.mark.parametrize("rows,cols,batch", [
+    (17, 32, 1), (16, 96, 2), (40, 31 * 32, 15), (33, 32 * 32, 16), (5, 33 * 32, 17), (47, 64 * 32, 31),
+    (16, 65 * 32, 33), (31, 512 * 32, 3),
+    (7168, 15 * 32, 5), (7153, 16 * 32, 16), (3600, 17 * 32, 19), (7185, 33 * 32, 2),
+    (9216, 13 * 32, 64), (9216, 13 * 32, 65),
+])
+def test_gemm_q4_0_few_tokens_bit_exact(backend, dev, orc, synth, rows, cols, batch):
+    rng = synth.rng_for(5180 + rows + cols + batch)
+    w = synth.q4_0_matrix(rng, rows, cols)
+    w2 = synth.q4_0_matrix(rng, rows, cols)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    x[batch - 1, :32] = 0.0  # a zero block in the last token
+    got = run_gemm(backend, dev, w, x, rows, cols, batch)
+    ref = oracle_gemm(orc, w, x, rows, cols, range(batch))
+    assert_bit_exact(got, ref, f"gemm {rows}x{cols} M={batch}")
+    bg = backend.HipBuffer.from_gguf(dev, w, backend.Q4_0, rows, cols)
+    bu = backend.HipBuffer.from_gguf(dev, w2, backend.Q4_0, rows, cols)
+    xb = backend.HipBuffer.from_host(dev, x.reshape(-1))
+    ab = backend.HipBuffer.alloc(dev, batch * rows)
+    dev.gemm_q4_0_geglu(bg, bu, xb, ab, rows, cols, batch)
+    dev.sync()
+    u = oracle_gemm(orc, w2, x, rows, cols, range(batch))
+    assert_bit_exact(ab.numpy().reshape(batch, rows), np.stack([orc.geglu(ref[m], u[m]) for m in range(batch)]),
+                     "geglu")
+
+
 def test_gemm_q4_0_qkv_geglu_any_rows(backend, dev, orc, synth):
     """The fused batched entries at row counts that are not multiples of 32
     or of 4: the k and v products then start off a 16-byte boundary of the
