@@ -22,6 +22,7 @@
 
 #include <math.h>
 
+#include "attn_common.h"
 #include "device.h"
 #include "exact_sum.h"
 #include "internal.h"
@@ -323,19 +324,6 @@ __global__ __launch_bounds__(512) void rope_kv_f16_kernel(float *__restrict__ qk
 // first (cache row = position % capacity).  Query head h reads kv head
 // h / (n_heads / n_kv_heads).
 
-__device__ __forceinline__ size_t cache_row_of(int t, int capacity) { return (size_t)(capacity > 0 ? t % capacity : t); }
-
-// The window: the last min(n_past + 1, limit) positions, limit = the cache
-// capacity or, below it, the sliding window (cuda.rs:2658-2697 sliding_window;
-// kernels.rs:1398-1404).  Cache rows stay position % capacity.
-__device__ __forceinline__ void attn_window(const int32_t *d_pos, int n_past_arg, int limit, int &window, int &start)
-{
-    const int n_past = d_pos ? *d_pos : n_past_arg;
-    const int count = n_past + 1;
-    window = (limit > 0 && count > limit) ? limit : count;
-    start = count - window;
-}
-
 // Scores: score[h][p] = (sum_d q_h[d] * k_{start+p}[d], from -0.0 in d
 // order) * scale.  Workgroup (tile of 64 positions, kv head) with one wave per
 // query head of the group: the K tile (64 rows x 512 B) is loaded with
@@ -429,8 +417,6 @@ constexpr int kKRow2 = kAttnHD * 2 + 16;  // padded K row in LDS, bytes
 
 // Native 4 and 2 x 32-bit vectors: copies of HIP's uint4 struct lower to
 // memcpy, which keeps an array of them in scratch memory instead of registers.
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 constexpr int kScoreT = 256;              // threads per score workgroup
 
 
@@ -829,104 +815,6 @@ __global__ __launch_bounds__(kScoreT) void attn_scores2_kernel(const float *__re
         }
     }
     if (p0 + p < window) scores[(size_t)(kvh * G + g) * capacity + p0 + p] = dot * scale;
-}
-
-// Prefill form of the scores: positions tiled absolutely, so one K tile
-// serves several query rows.  Workgroup (tile of 64 positions T0.., kv head,
-// block of RB = 8 / G consecutive query rows): the tile's K rows are staged
-// in LDS once, then wave w runs row w / G, head w % G of the group, lane p
-// the chain of position T0 + p when the row's window holds it (the same
-// arithmetic as attn_scores2_kernel: q . k from -0.0 in dim order, one
-// product and one add per dim, times scale), stored at the position's index
-// in that row's window.  Row z's position is n_past0 + z; t_lo is row 0's
-// window start.
-constexpr int kSRowsW = 8;  // waves per workgroup
-template <int G>
-__global__ __launch_bounds__(64 * kSRowsW) void attn_scores_rows_kernel(const float *__restrict__ q_in, int q_stride,
-                                                                      const uint16_t *__restrict__ k_cache,
-                                                                      int n_past0, int rows, int n_heads,
-                                                                      int n_kv_heads, float scale, int capacity,
-                                                                      int wlimit, int t_lo, float *__restrict__ scores)
-{
-    constexpr int HD = kAttnHD, P = kScoreP, RB = kSRowsW / G, NT = 64 * kSRowsW;
-    __shared__ __align__(16) float q_s[RB * G][HD];
-    __shared__ __align__(16) uint8_t k_s[P * kKRow2];
-    // row blocks in reverse order: the latest rows, with the most tiles, are
-    // dispatched first, so the launch does not end on them
-    const int T0 = t_lo + (int)blockIdx.x * P, kvh = blockIdx.y, tid = threadIdx.x;
-    const int z0 = ((int)gridDim.z - 1 - (int)blockIdx.z) * RB;
-    const int zl = (z0 + RB < rows ? z0 + RB : rows) - 1;  // the block's last row
-    int win0, start0, winl, startl;
-    attn_window(nullptr, n_past0 + z0, wlimit, win0, start0);
-    attn_window(nullptr, n_past0 + zl, wlimit, winl, startl);
-    const int pos_l = n_past0 + zl;
-    if (T0 > pos_l || T0 + P - 1 < start0) return;  // no row of the block has a position in this tile
-    const size_t kv_dim = (size_t)n_kv_heads * HD;
-    // K tile: 2048 chunks of 16 B (positions past the block's newest one
-    // reload that row; their scores are not stored)
-    constexpr int kChunks = P * (HD * 2 / 16), kPer = kChunks / NT;
-    u32x4 tmp[kPer];
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-        const int c = k * NT + tid, r = c >> 5;
-        const int t = T0 + r <= pos_l ? T0 + r : pos_l;
-        tmp[k] = reinterpret_cast<const u32x4 *>(k_cache + cache_row_of(t, capacity) * kv_dim + (size_t)kvh * HD)[c & 31];
-    }
-    // q of the block's rows and the group's heads: RB*G*HD floats, float4 each
-    for (int i = tid; i < RB * G * HD / 4; i += NT) {
-        const int w = i / (HD / 4), e = i % (HD / 4), r = w / G, g = w % G;
-        const int z = z0 + r < rows ? z0 + r : rows - 1;
-        reinterpret_cast<float4 *>(q_s[w])[e] =
-            reinterpret_cast<const float4 *>(q_in + (size_t)z * q_stride + (size_t)(kvh * G + g) * HD)[e];
-    }
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-        const int c = k * NT + tid, r = c >> 5;
-        *reinterpret_cast<u32x4 *>(k_s + r * kKRow2 + (c & 31) * 16) = tmp[k];
-    }
-    __syncthreads();
-    const int w = tid >> 6, p = tid & 63;
-    if (w >= RB * G) return;
-    const int r = w / G, g = w % G, z = z0 + r, t = T0 + p;
-    if (z >= rows) return;
-    int window, start;
-    attn_window(nullptr, n_past0 + z, wlimit, window, start);
-    const u32x4 *krow = reinterpret_cast<const u32x4 *>(k_s + p * kKRow2);
-    const float4 *qg = reinterpret_cast<const float4 *>(q_s[w]);
-    float nz;
-    asm volatile("v_mov_b32 %0, 0x80000000" : "=v"(nz));
-    float dot = -0.0f;
-    constexpr int kSteps = HD / 32;
-    u32x4 kw[2][4];
-    float4 qa[2][8];
-    auto fetch = [&](int st, int b) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            kw[b][u] = krow[4 * st + u];
-            qa[b][2 * u] = qg[2 * (4 * st + u)];
-            qa[b][2 * u + 1] = qg[2 * (4 * st + u) + 1];
-        }
-    };
-    fetch(0, 0);
-#pragma unroll
-    for (int st = 0; st < kSteps; ++st) {
-        const int b = st & 1;
-        if (st + 1 < kSteps) fetch(st + 1, b ^ 1);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const u32x4 wv = kw[b][u];
-            const uint32_t wd[4] = {wv.x, wv.y, wv.z, wv.w};
-            const float qv[8] = {qa[b][2 * u].x, qa[b][2 * u].y, qa[b][2 * u].z, qa[b][2 * u].w,
-                                 qa[b][2 * u + 1].x, qa[b][2 * u + 1].y, qa[b][2 * u + 1].z, qa[b][2 * u + 1].w};
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const _Float16 kh = __builtin_bit_cast(_Float16, (uint16_t)(wd[e >> 1] >> (16 * (e & 1))));
-                dot = dot + __builtin_fmaf(qv[e], (float)kh, nz);
-            }
-        }
-    }
-    if (t >= start && t < start + window)
-        scores[((size_t)z * n_heads + kvh * G + g) * capacity + (t - start)] = dot * scale;
 }
 
 // Softmax and weighted values, query head h, dims [32*ds, 32*ds + 32) per
@@ -1415,165 +1303,6 @@ __global__ __launch_bounds__(kSplitT) void attn_split_kernel(const float *__rest
     }
 }
 
-// Prefill form of attn_softmax_v_kernel: one workgroup per (query row, kv
-// head), thread d = output dim d of each of the group's G query heads.  Each
-// row's arithmetic is the decode form's -- per head the max over the window,
-// e_p = expf(s_p - max), the ordered exp sum, p_p = e_p * (1/sum), out[d] =
-// 0 + p_0 v_0[d] + p_1 v_1[d] + ... in order -- but the softmax is formed
-// once per head rather than once per 32-dim slice, and each thread runs its
-// dim's chains, one per head of the group, over V rows read straight from
-// the cache: every V load feeds G chains, and the next 32 positions' loads
-// are in flight while the current 32 are added.  The decode form spreads
-// one long row over eight workgroups to cut its latency; a prefill chunk has
-// rows enough to fill the GPU this way.  Windows up to kRowsSvMax positions
-// (one exact block sum per head) and groups of G <= kRowsSvG heads (a
-// compile-time count, so the per-position work has no head loop or test).
-// Dynamic LDS: the group's weights, G rows of `span` floats (the launch's
-// widest window) at a stride of a multiple of 4 floats, then span flag bytes.
-constexpr int kRowsSvMax = mrml_xsum::kMaxPerThread * kAttnHD;  // 4096
-constexpr int kRowsSvG = 4;
-constexpr int kRowsSvB = 32;  // positions per load batch
-inline int rows_sv_stride(int span) { return (span + 3) & ~3; }
-inline size_t rows_sv_lds(int g, int span)
-{
-    return (size_t)g * rows_sv_stride(span) * sizeof(float) + ((span + 15) & ~15);
-}
-
-// SHORT (windows up to 4 * kAttnHD): thread d takes positions 4d..4d+3, its
-// exps stay in registers for the register form of the exact sum.
-template <int G, bool SHORT>
-__global__ __launch_bounds__(kAttnHD) void attn_softmax_v_rows_kernel(const float *__restrict__ scores,
-                                                                      const uint16_t *__restrict__ v_cache,
-                                                                      int n_past0, int n_heads, int n_kv_heads,
-                                                                      int capacity, int wlimit, int expf_fused,
-                                                                      float *__restrict__ out, int span)
-{
-    constexpr int HD = kAttnHD, B = kRowsSvB;
-    extern __shared__ __align__(16) float e_dyn[];  // [G][span] weights, then span flag bytes
-    __shared__ float red[HD / 64];
-    __shared__ uint64_t exp_tab[32];
-    // rows in reverse order: the longest windows are dispatched first, so the
-    // launch does not end on them
-    const int kvh = blockIdx.x, z = (int)gridDim.y - 1 - (int)blockIdx.y, d = threadIdx.x, stride = (span + 3) & ~3;
-    uint8_t *flags = reinterpret_cast<uint8_t *>(e_dyn + (size_t)G * stride);
-    auto e_s = [&](int g) { return e_dyn + (size_t)g * stride; };
-    int window, start;
-    attn_window(nullptr, n_past0 + z, wlimit, window, start);
-    if (d < 32) exp_tab[d] = mrml_libm::kExpfT.t[d];
-    const bool fused = expf_fused != 0;
-    if constexpr (SHORT) {
-        __shared__ mrml_xsum::Shared4 xs4;
-        const int p = 4 * d;
-#pragma unroll 1
-        for (int g = 0; g < G; ++g) {
-            const float *sc = scores + ((size_t)z * n_heads + kvh * G + g) * capacity;
-            float sv[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) sv[i] = p + i < window ? sc[p + i] : -INFINITY;
-            float mx = fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]));  // the max is exact in any order
-            mx = wave_max_f32(mx);
-            if ((d & 63) == 0) red[d >> 6] = mx;
-            __syncthreads();
-            mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-            float e[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) e[i] = p + i < window ? mrml_libm::expf_t(sv[i] - mx, fused, exp_tab) : 0.0f;
-            // (its first barrier also orders every thread's read of red
-            // before the next head rewrites it)
-            const float sum = mrml_xsum::block_seq_sum_nonneg4(make_float4(e[0], e[1], e[2], e[3]), window, xs4);
-            const float inv = sum > 0.0f ? 1.0f / sum : 1.0f;
-            float *eg = e_s(g);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (p + i < window) eg[p + i] = sum > 0.0f ? e[i] * inv : e[i];
-        }
-    } else {
-#pragma unroll 1
-    for (int g = 0; g < G; ++g) {
-        const float *sc = scores + ((size_t)z * n_heads + kvh * G + g) * capacity;
-        float mx = -INFINITY;  // the max is exact in any order
-        for (int p = d; p < window; p += HD) mx = fmaxf(mx, sc[p]);
-        mx = wave_max_f32(mx);
-        if ((d & 63) == 0) red[d >> 6] = mx;
-        __syncthreads();
-        mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-        float *eg = e_s(g);
-        for (int p = d; p < window; p += HD) eg[p] = mrml_libm::expf_t(sc[p] - mx, fused, exp_tab);
-        __syncthreads();  // also: every thread has read red before the next head rewrites it
-        __shared__ mrml_xsum::Shared xs;
-        const float sum = mrml_xsum::block_seq_sum_nonneg(eg, window, flags, xs);  // ends with a barrier
-        if (sum > 0.0f) {
-            const float inv = 1.0f / sum;
-            for (int p = d; p < window; p += HD) eg[p] = eg[p] * inv;
-        }
-    }
-    }
-    __syncthreads();
-    const size_t kv_dim = (size_t)n_kv_heads * HD;
-    const uint16_t *vb = v_cache + (size_t)kvh * HD + d;
-    float acc[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g) acc[g] = 0.0f;
-    int row = (int)cache_row_of(start, capacity);  // the window's rows are consecutive modulo capacity
-    // unconditional loads (row stays a cache row; positions past the window
-    // are skipped by add), so all B of them are issued before any is used
-    auto load = [&](float (&v)[B], int) {
-        uint16_t raw[B];
-#pragma unroll
-        for (int k = 0; k < B; ++k) {
-            raw[k] = vb[(size_t)row * kv_dim];
-            row = row + 1 == capacity ? 0 : row + 1;
-        }
-#pragma unroll
-        for (int k = 0; k < B; ++k) v[k] = f16_bits_to_f32(raw[k]);
-    };
-    // a batch inside the window: each head's weights read four positions at
-    // a time (float4 broadcasts), no per-position test
-    auto add_full = [&](const float (&v)[B], int t0) {
-#pragma unroll
-        for (int i = 0; i < B / 4; ++i) {
-            float4 e4[G];
-#pragma unroll
-            for (int g = 0; g < G; ++g) e4[g] = reinterpret_cast<const float4 *>(e_s(g) + t0)[i];
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                acc[g] = acc[g] + e4[g].x * v[4 * i];
-                acc[g] = acc[g] + e4[g].y * v[4 * i + 1];
-                acc[g] = acc[g] + e4[g].z * v[4 * i + 2];
-                acc[g] = acc[g] + e4[g].w * v[4 * i + 3];
-            }
-        }
-    };
-    // the window's last, partial batch
-    auto add_part = [&](const float (&v)[B], int t0) {
-#pragma unroll
-        for (int k = 0; k < B; ++k) {
-            if (t0 + k < window) {
-#pragma unroll
-                for (int g = 0; g < G; ++g) acc[g] = acc[g] + e_s(g)[t0 + k] * v[k];
-            }
-        }
-    };
-    float va[B], vb2[B];
-    load(va, 0);
-    int t0 = 0;
-    for (; t0 + 2 * B <= window; t0 += 2 * B) {
-        load(vb2, t0 + B);  // in flight while va is added
-        add_full(va, t0);
-        load(va, t0 + 2 * B);
-        add_full(vb2, t0 + B);
-    }
-    if (t0 + B <= window) {
-        load(vb2, t0 + B);
-        add_full(va, t0);
-        add_part(vb2, t0 + B);
-    } else {
-        add_part(va, t0);
-    }
-#pragma unroll
-    for (int g = 0; g < G; ++g) out[((size_t)z * n_heads + kvh * G + g) * HD + d] = acc[g];
-}
-
 // Merges the tiles of head blockIdx.x (thread d = output dim d), in tile
 // order, and writes out (nullable) and the Q8_0 pack (nullable) of the
 // n_heads*256 output.
@@ -1905,75 +1634,6 @@ int launch_attn_decode_f16(mrml_hip_ctx *ctx, const float *q, const uint16_t *k_
     return launch_softmax_v(ctx, scores, v_cache, out, pack, d_pos, n_past, n_heads, n_kv_heads, capacity, wlimit);
 }
 
-// Attention of `rows` queries at consecutive positions n_past0, n_past0+1, ...
-// (the prefill of a chunk whose K/V rows are already in the cache): query row
-// r starts r * q_stride floats into q (q_stride = the stacked q|k|v width
-// when q is the projection itself); output row r (n_heads*head_dim f32) goes
-// to out.  Each row's arithmetic is that of launch_attn_decode_f16 at its
-// position with the same sliding window.  scratch holds rows * n_heads *
-// capacity floats.  Groups of up to 8 query heads per kv head.
-int launch_attn_rows_f16(mrml_hip_ctx *ctx, const float *q, int q_stride, const uint16_t *k_cache,
-                         const uint16_t *v_cache, float *out, int n_past0, int rows, int n_heads, int n_kv_heads,
-                         float scale, int capacity, void *scratch, int sliding_window)
-{
-    float *scores = reinterpret_cast<float *>(scratch);
-    const int wlimit = attn_window_limit(capacity, sliding_window);
-    // score tiles up to the widest row window (the host knows every row's position)
-    const int span = std::min(wlimit, n_past0 + rows);
-    const dim3 sgrid((span + kScoreP - 1) / kScoreP, n_kv_heads, rows);
-    if (attn_rope_ok(n_heads, n_kv_heads) && (q_stride % 4 != 0 || ((uintptr_t)q & 15) != 0)) {
-        // q rows that float4 reads cannot reach: one workgroup per row and tile
-        hipLaunchKernelGGL(attn_scores2_kernel<false>, sgrid, dim3(kScoreT), 0, ctx->stream, q,
-                           const_cast<uint16_t *>(k_cache), (uint16_t *)nullptr, (const int32_t *)nullptr, n_past0,
-                           n_heads, n_kv_heads, scale, capacity, wlimit, RopeArgs{}, scores, q_stride);
-        if (int rc = check_launch(ctx, "attn_scores2_kernel")) return rc;
-    } else if (attn_rope_ok(n_heads, n_kv_heads)) {
-        // positions tiled absolutely from row 0's window start to the last
-        // row's position, 8 / G rows a workgroup
-        const int g = n_heads / n_kv_heads, rb = kSRowsW / g;
-        const int count0 = n_past0 + 1, t_lo = count0 > wlimit ? count0 - wlimit : 0, t_hi = n_past0 + rows - 1;
-        const dim3 rgrid((unsigned)((t_hi - t_lo + kScoreP) / kScoreP), (unsigned)n_kv_heads,
-                         (unsigned)((rows + rb - 1) / rb));
-#define SCORES_ROWS(G)                                                                                          \
-    hipLaunchKernelGGL(attn_scores_rows_kernel<G>, rgrid, dim3(64 * kSRowsW), 0, ctx->stream, q, q_stride,       \
-                       k_cache, n_past0, rows, n_heads, n_kv_heads, scale, capacity, wlimit, t_lo, scores)
-        switch (g) {
-        case 1: SCORES_ROWS(1); break;
-        case 2: SCORES_ROWS(2); break;
-        case 3: SCORES_ROWS(3); break;
-        default: SCORES_ROWS(4); break;
-        }
-#undef SCORES_ROWS
-        if (int rc = check_launch(ctx, "attn_scores_rows_kernel")) return rc;
-    } else {
-        hipLaunchKernelGGL(attn_scores_kernel, sgrid, dim3(64 * (n_heads / n_kv_heads)), 0, ctx->stream, q, k_cache,
-                           (const int32_t *)nullptr, n_past0, n_heads, n_kv_heads, scale, capacity, wlimit, scores,
-                           q_stride);
-        if (int rc = check_launch(ctx, "attn_scores_kernel")) return rc;
-    }
-    // the rows form where its dynamic LDS stays within 60 KiB; with the
-    // kernel's static LDS (mrml_xsum::Shared, red, exp_tab: about 8.6 KB)
-    // a launch takes up to about 69 KB, within gfx950's 160 KiB a workgroup
-    if (span <= kRowsSvMax && n_heads / n_kv_heads <= kRowsSvG &&
-        rows_sv_lds(n_heads / n_kv_heads, span) <= (size_t)60 << 10) {
-#define ROWS_SV(G, S)                                                                                           \
-    hipLaunchKernelGGL((attn_softmax_v_rows_kernel<G, S>), dim3(n_kv_heads, rows), dim3(kAttnHD),                \
-                       rows_sv_lds(n_heads / n_kv_heads, span), ctx->stream, scores, v_cache, n_past0, n_heads,   \
-                       n_kv_heads, capacity, wlimit, (int)host_expf_fused(), out, span)
-        const bool sh = span <= 4 * kAttnHD;
-        switch (n_heads / n_kv_heads) {
-        case 1: if (sh) ROWS_SV(1, true); else ROWS_SV(1, false); break;
-        case 2: if (sh) ROWS_SV(2, true); else ROWS_SV(2, false); break;
-        case 3: if (sh) ROWS_SV(3, true); else ROWS_SV(3, false); break;
-        default: if (sh) ROWS_SV(4, true); else ROWS_SV(4, false); break;
-        }
-#undef ROWS_SV
-        return check_launch(ctx, "attn_softmax_v_rows_kernel");
-    }
-    return launch_softmax_v(ctx, scores, v_cache, out, nullptr, nullptr, n_past0, n_heads, n_kv_heads, capacity, wlimit,
-                            rows);
-}
-
 // The decode step's attention with RoPE and the K/V append in the scores
 // kernel: qkv is the raw stacked q|k|v vector.  Needs n_heads / n_kv_heads
 // <= 4 (attn_rope_ok).
@@ -2006,12 +1666,11 @@ bool attn_tuned(int n_heads, int n_kv_heads, int head_dim, int k_fmt, int v_fmt)
     return head_dim == kAttnHD && k_fmt == 0 && v_fmt == 0 && n_kv_heads > 0 && n_heads / n_kv_heads <= 8;
 }
 
-int launch_attn_any(mrml_hip_ctx *ctx, const float *q, int q_stride, const void *k_cache, const void *v_cache,
-                    float *out, void *pack, const int32_t *d_pos, int n_past0, int rows, int n_heads, int n_kv_heads,
-                    int head_dim, int k_fmt, int v_fmt, float scale, int capacity, void *scratch, int sliding_window)
+// Scores over K rows of format k_fmt, one workgroup a (64 positions, kv head, row).
+static int launch_any_scores(mrml_hip_ctx *ctx, const float *q, int q_stride, const void *k_cache, const int32_t *d_pos,
+                             int n_past0, int rows, int n_heads, int n_kv_heads, int head_dim, int k_fmt, float scale,
+                             int capacity, int wlimit, float *scores)
 {
-    float *scores = reinterpret_cast<float *>(scratch);
-    const int wlimit = attn_window_limit(capacity, sliding_window);
     // score tiles up to the widest row window (every tile when the position is on the device)
     const int span = d_pos ? wlimit : std::min(wlimit, n_past0 + rows);
     const dim3 sgrid((span + kAnyP - 1) / kAnyP, n_kv_heads, rows);
@@ -2027,9 +1686,55 @@ int launch_attn_any(mrml_hip_ctx *ctx, const float *q, int q_stride, const void 
     else
         SC_LAUNCH(0);
 #undef SC_LAUNCH
-    if (int rc = check_launch(ctx, "attn_scores_any_kernel")) return rc;
-    return launch_softmax_v(ctx, scores, v_cache, out, pack, d_pos, n_past0, n_heads, n_kv_heads, capacity, wlimit,
-                            rows, head_dim, v_fmt);
+    return check_launch(ctx, "attn_scores_any_kernel");
+}
+
+int launch_attn_any(mrml_hip_ctx *ctx, const float *q, const void *k_cache, const void *v_cache, float *out, void *pack,
+                    const int32_t *d_pos, int n_past, int n_heads, int n_kv_heads, int head_dim, int k_fmt, int v_fmt,
+                    float scale, int capacity, void *scratch, int sliding_window)
+{
+    float *scores = reinterpret_cast<float *>(scratch);
+    const int wlimit = attn_window_limit(capacity, sliding_window);
+    if (int rc = launch_any_scores(ctx, q, 0, k_cache, d_pos, n_past, 1, n_heads, n_kv_heads, head_dim, k_fmt, scale,
+                                   capacity, wlimit, scores))
+        return rc;
+    return launch_softmax_v(ctx, scores, v_cache, out, pack, d_pos, n_past, n_heads, n_kv_heads, capacity, wlimit, 1,
+                            head_dim, v_fmt);
+}
+
+// Attention of `rows` queries at consecutive positions n_past0, n_past0+1, ...
+// (the prefill of a chunk whose K/V rows are already in the cache): query row
+// r starts r * q_stride floats into q (q_stride = the stacked q|k|v width
+// when q is the projection itself); output row r (n_heads*head_dim f32) goes
+// to out.  Each row's arithmetic is the decode form's at its position with
+// the same sliding window.  scratch holds rows * n_heads * capacity floats.
+int launch_attn_rows(mrml_hip_ctx *ctx, const float *q, int q_stride, const void *k_cache, const void *v_cache,
+                     float *out, int n_past0, int rows, int n_heads, int n_kv_heads, int head_dim, int k_fmt, int v_fmt,
+                     float scale, int capacity, void *scratch, int sliding_window)
+{
+    float *scores = reinterpret_cast<float *>(scratch);
+    const int wlimit = attn_window_limit(capacity, sliding_window), span = std::min(wlimit, n_past0 + rows);
+    if (int rc = k_fmt == 0
+                     ? launch_attn_rows_scores(ctx, q, q_stride, (const uint16_t *)k_cache, n_past0, rows, n_heads,
+                                               n_kv_heads, head_dim, scale, capacity, wlimit, scores)
+                     : launch_any_scores(ctx, q, q_stride, k_cache, nullptr, n_past0, rows, n_heads, n_kv_heads,
+                                         head_dim, k_fmt, scale, capacity, wlimit, scores))
+        return rc;
+    // The decode form's workgroup adds 32 dims of one row at 4.7 ns a
+    // position, the rows form's waves need company for that: while the decode
+    // form's workgroups are all resident at once (three or four a CU) and its
+    // repeated softmax is not what they spend their time on, it is the faster.
+    // Measured (us, decode form / rows form, 8 heads): 8 rows x 256 dims (512
+    // workgroups) at 300 positions 20 / 22, at 3000 75 / 83; 12 rows (768) at
+    // 300 25 / 22; 60 rows x 64 dims (960) at 1000 54 / 66; 20 rows x 256
+    // (1280) at 512 47 / 44; 32 rows (2048) at 100 44 / 19.
+    const int64_t wgs = (int64_t)rows * n_heads * (head_dim / kSVD);
+    if (wgs <= 512 || (wgs <= 1024 && span > 512) ||
+        !attn_rows_v_ok(n_kv_heads, head_dim, v_fmt, capacity))
+        return launch_softmax_v(ctx, scores, v_cache, out, nullptr, nullptr, n_past0, n_heads, n_kv_heads, capacity,
+                                wlimit, rows, head_dim, v_fmt);
+    return launch_attn_rows_softmax_v(ctx, scores, v_cache, out, n_past0, rows, n_heads, n_kv_heads, head_dim, v_fmt,
+                                      capacity, wlimit);
 }
 
 int launch_rope_kv_any(mrml_hip_ctx *ctx, float *qkv, void *k_cache, void *v_cache, int pos, int n_heads,

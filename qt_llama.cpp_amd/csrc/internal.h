@@ -213,21 +213,28 @@ int launch_attn_decode_f16(mrml_hip_ctx *ctx, const float *q, const uint16_t *k_
 bool attn_rope_ok(int n_heads, int n_kv_heads);
 // `rows` batched queries at positions n_past0.., query rows q_stride floats
 // apart (prefill); scratch of rows * attn_scratch_bytes(n_heads, capacity).
-// Groups of up to 8 query heads per kv head.
-int launch_attn_rows_f16(mrml_hip_ctx *ctx, const float *q, int q_stride, const uint16_t *k_cache,
-                         const uint16_t *v_cache, float *out, int n_past0, int rows, int n_heads, int n_kv_heads,
-                         float scale, int capacity, void *scratch, int sliding_window = -1);
+// Any shape and format that attn_any_ok takes.
+int launch_attn_rows(mrml_hip_ctx *ctx, const float *q, int q_stride, const void *k_cache, const void *v_cache,
+                     float *out, int n_past0, int rows, int n_heads, int n_kv_heads, int head_dim, int k_fmt, int v_fmt,
+                     float scale, int capacity, void *scratch, int sliding_window);
+// Its parts in attn_rows.hip: scores over f16 K rows; softmax and weighted sum
+// (caches that attn_rows_v_ok says a buffer descriptor reaches).
+int launch_attn_rows_scores(mrml_hip_ctx *ctx, const float *q, int q_stride, const uint16_t *k_cache, int n_past0,
+                            int rows, int n_heads, int n_kv_heads, int head_dim, float scale, int capacity, int wlimit,
+                            float *scores);
+bool attn_rows_v_ok(int n_kv_heads, int head_dim, int v_fmt, int capacity);
+int launch_attn_rows_softmax_v(mrml_hip_ctx *ctx, float *scores, const void *v_cache, float *out, int n_past0, int rows,
+                               int n_heads, int n_kv_heads, int head_dim, int v_fmt, int capacity, int wlimit);
 // Attention over caches of any head size (a multiple of 32 up to 512),
 // groups of up to 16 and the KV formats 0 (f16), 1 (Q8_0), 2 (Q4_0):
-// `rows` queries at positions n_past0.. (or d_pos, rows = 1), the arithmetic
-// of the CPU loop over KvCacheRow::dot_head / add_head_scaled.  scratch of
-// rows * attn_scratch_bytes(n_heads, capacity).
+// one query at position n_past (or *d_pos), the arithmetic of the CPU loop
+// over KvCacheRow::dot_head / add_head_scaled.  scratch of
+// attn_scratch_bytes(n_heads, capacity).
 bool attn_any_ok(int n_heads, int n_kv_heads, int head_dim);
 bool attn_tuned(int n_heads, int n_kv_heads, int head_dim, int k_fmt, int v_fmt);
-int launch_attn_any(mrml_hip_ctx *ctx, const float *q, int q_stride, const void *k_cache, const void *v_cache,
-                    float *out, void *pack, const int32_t *d_pos, int n_past0, int rows, int n_heads, int n_kv_heads,
-                    int head_dim, int k_fmt, int v_fmt, float scale, int capacity, void *scratch,
-                    int sliding_window = -1);
+int launch_attn_any(mrml_hip_ctx *ctx, const float *q, const void *k_cache, const void *v_cache, float *out, void *pack,
+                    const int32_t *d_pos, int n_past, int n_heads, int n_kv_heads, int head_dim, int k_fmt, int v_fmt,
+                    float scale, int capacity, void *scratch, int sliding_window);
 // RoPE of `rows` stacked q|k|v rows at positions pos.. and their K/V appended
 // to caches of formats k_fmt / v_fmt at cache rows (pos + i + cache_shift) %
 // capacity (f16 caches: launch_rope_kv_f16 alone).

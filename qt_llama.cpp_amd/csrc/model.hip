@@ -281,7 +281,7 @@ static int attn_exact(mrml_hip_ctx *ctx, const float *q, const uint16_t *k_cache
     void *part = workspace(ctx, attn_scratch_bytes(n_heads, capacity));
     if (!part) return MRML_HIP_E_ALLOC;
     if (!attn_tuned(n_heads, n_kv_heads, head_dim, k_format, v_format))
-        return launch_attn_any(ctx, q, 0, k_cache, v_cache, out, pack, d_pos, n_past, 1, n_heads, n_kv_heads,
+        return launch_attn_any(ctx, q, k_cache, v_cache, out, pack, d_pos, n_past, n_heads, n_kv_heads,
                                head_dim, k_format, v_format, scale, capacity, part, sliding_window);
     return launch_attn_decode_f16(ctx, q, k_cache, v_cache, out, pack, d_pos, n_past, n_heads, n_kv_heads, scale,
                                   capacity, part, sliding_window);
@@ -368,16 +368,10 @@ int mrml_hip_attention_prefill(mrml_hip_ctx *ctx, const float *q, int32_t q_stri
     const int rn = (int)std::max<size_t>(1, std::min<size_t>(std::min(batch, 65535), kPrefillScoreBytes / per));
     void *part = workspace(ctx, (size_t)rn * per);
     if (!part) return MRML_HIP_E_ALLOC;
-    const bool tuned = attn_tuned(n_heads, n_kv_heads, head_dim, k_format, v_format);
     for (int r0 = 0; r0 < batch; r0 += rn) {
-        const int n = std::min(rn, batch - r0);
-        const int rc = tuned ? launch_attn_rows_f16(ctx, q + (size_t)r0 * q_stride, q_stride, k_cache, v_cache,
-                                                    out + r0 * qd, cache_start + r0, n, n_heads, n_kv_heads, scale,
-                                                    capacity, part, sliding_window)
-                             : launch_attn_any(ctx, q + (size_t)r0 * q_stride, q_stride, k_cache, v_cache,
-                                               out + r0 * qd, nullptr, nullptr, cache_start + r0, n, n_heads,
-                                               n_kv_heads, head_dim, k_format, v_format, scale, capacity, part,
-                                               sliding_window);
+        const int rc = launch_attn_rows(ctx, q + (size_t)r0 * q_stride, q_stride, k_cache, v_cache, out + r0 * qd,
+                                        cache_start + r0, std::min(rn, batch - r0), n_heads, n_kv_heads, head_dim,
+                                        k_format, v_format, scale, capacity, part, sliding_window);
         if (rc) return rc;
     }
     return MRML_HIP_OK;
@@ -708,9 +702,9 @@ int mrml_hip_gemma2_prefill(mrml_hip_ctx *ctx, mrml_hip_gemma2 *m, const int32_t
                     STEP(launch_rope_kv_f16(ctx, qi, kc, vc, nullptr, p0 + i, c.n_heads, c.n_kv_heads, c.head_dim,
                                             c.rope_base, 1.0f, c.ctx_len, m->rope_table, c.ctx_len, 1, 0,
                                             m->rope_freqs));
-                    STEP(launch_attn_rows_f16(ctx, qi, (int)qkvd, kc, vc, m->pf_attn + (size_t)i * qd, p0 + i, 1,
-                                              c.n_heads, c.n_kv_heads, c.attn_scale, c.ctx_len, m->pf_scores,
-                                              layer_window(c, l)));
+                    STEP(launch_attn_rows(ctx, qi, (int)qkvd, kc, vc, m->pf_attn + (size_t)i * qd, p0 + i, 1,
+                                          c.n_heads, c.n_kv_heads, c.head_dim, 0, 0, c.attn_scale, c.ctx_len,
+                                          m->pf_scores, layer_window(c, l)));
                 }
             } else {
                 // every token's rotated k and v enter the cache before any token
@@ -719,10 +713,10 @@ int mrml_hip_gemma2_prefill(mrml_hip_ctx *ctx, mrml_hip_gemma2 *m, const int32_t
                                         c.rope_base, 1.0f, c.ctx_len, m->rope_table, c.ctx_len, n, 0,
                                         m->rope_freqs));
                 for (int r0 = 0, rn = prefill_attn_rows(c); r0 < n; r0 += rn)
-                    STEP(launch_attn_rows_f16(ctx, m->pf_qkv + (size_t)r0 * qkvd, (int)qkvd, kc, vc,
-                                              m->pf_attn + (size_t)r0 * qd, p0 + r0, std::min(rn, n - r0),
-                                              c.n_heads, c.n_kv_heads, c.attn_scale, c.ctx_len, m->pf_scores,
-                                              layer_window(c, l)));
+                    STEP(launch_attn_rows(ctx, m->pf_qkv + (size_t)r0 * qkvd, (int)qkvd, kc, vc,
+                                          m->pf_attn + (size_t)r0 * qd, p0 + r0, std::min(rn, n - r0), c.n_heads,
+                                          c.n_kv_heads, c.head_dim, 0, 0, c.attn_scale, c.ctx_len, m->pf_scores,
+                                          layer_window(c, l)));
             }
             STEP(gemm_rows(ctx, m, L.wo, m->pf_attn, m->pf_o, c.dim, qd, n));
             STEP(launch_residual_rms_norm(ctx, m->pf_o, L.post_attn_norm, h, h, L.ffn_norm, c.eps, xn, nullptr, c.dim,

@@ -184,6 +184,52 @@ def test_attention_prefill_any(backend, dev, orc, nh, nkv, hd, kf, vf):
         assert_bits(got[i], ref, f"row {i}")
 
 
+# Batches that take the many-row kernels (attn_rows.hip), by what can go wrong
+# there: each weighted-sum form (chain rows x dims a wave: 4x2, 4x1, 2x1, 1x1)
+# at every value format, groups of 3, head sizes whose last 64-dim slice is
+# ragged, rows whose windows start or end apart (sliding windows, a window of
+# one position), the ring's end inside the window, capacities below a tile,
+# softmax rows of one chunk and of several (1024 rows x heads and more past
+# 1024 positions), and the decode form's side of the line.
+@pytest.mark.parametrize("nh,nkv,hd,kf,vf,cap,sw,start,batch", [
+    (8, 4, 256, 0, 0, 1024, None, 300, 300),   # 4x1, tail batches of every length
+    (8, 4, 256, 0, 0, 2048, None, 0, 513),     # 4x2, from position 0
+    (8, 4, 256, 0, 0, 256, None, 500, 77),     # 2x1, the ring wrapped
+    (16, 2, 128, 0, 0, 4096, None, 1030, 70),  # softmax in chunks
+    (12, 4, 96, 0, 0, 512, 100, 290, 200),     # group of 3, ragged slice, sliding
+    (4, 4, 64, 0, 0, 512, 1, 40, 300),         # one position a window
+    (4, 4, 32, 0, 0, 40, 7, 100, 300),         # a capacity below a tile
+    (8, 1, 512, 0, 0, 640, 333, 400, 90),      # group of 8, 512 dims
+    (8, 4, 256, 1, 2, 512, 200, 450, 150),     # quantised, 4x2, the ring's end inside
+    (8, 2, 128, 2, 1, 512, None, 200, 150),
+    (4, 4, 64, 1, 1, 256, 50, 100, 170),       # quantised, 1x1
+    (6, 2, 96, 2, 2, 300, 130, 280, 130),      # 2x1
+    (8, 4, 256, 0, 0, 512, None, 100, 8),      # decode form (512 workgroups)
+    (8, 4, 256, 0, 0, 512, None, 100, 9),
+])
+def test_attention_prefill_many_rows(backend, dev, orc, nh, nkv, hd, kf, vf, cap, sw, start, batch):
+    kvd, qd = nkv * hd, nh * hd
+    rng = np.random.default_rng(8250 + hd + cap + batch)
+    kx = rng.standard_normal((cap, kvd), dtype=np.float32)
+    vx = rng.standard_normal((cap, kvd), dtype=np.float32)
+    if cap == 512 and kf == 0 and vf == 0:
+        # outside the earliest row's window: the row must not meet it (0 * inf)
+        vx[(start + batch - 1) % cap, 0] = np.inf
+    kc, vc = cache_bytes(orc, kx, kf), cache_bytes(orc, vx, vf)
+    stride = qd + 2 * kvd + (1 if hd == 96 else 0)  # q rows off 16 bytes too
+    q = (rng.standard_normal(batch * stride) * 0.5).astype(np.float32)
+    qb, kb, vb = backend.HipBuffer.from_host(dev, q), upload_cache(backend, dev, kc), upload_cache(backend, dev, vc)
+    out = backend.HipBuffer.alloc(dev, batch * qd)
+    scale = float(np.float32(1.0 / np.sqrt(hd)))
+    print(f"\n[prefill many rows] heads {nh}/{nkv} hd {hd} formats {kf}/{vf} batch {batch}", flush=True)
+    dev.attention_prefill(qb, kb, vb, out, start, batch, nh, nkv, hd, scale, sw, cap, kf, vf, q_stride=stride)
+    dev.sync()
+    got = out.numpy().reshape(batch, qd)
+    for i in sorted({*range(4), batch // 3, batch // 2, *range(batch - 5, batch)}):
+        ref = oracle_rows(orc, q[i * stride:i * stride + qd], kc, vc, start + i, sw, cap, nh, nkv, hd, scale, kf, vf)
+        assert_bits(got[i], ref, f"row {i}")
+
+
 @pytest.mark.parametrize("hd,kf,vf", [(256, 0, 0), (128, 1, 1)])
 def test_attention_past_131072(backend, dev, orc, hd, kf, vf):
     """Capacities past 2^17 (the reference's default max_context is 256000,
