@@ -37,48 +37,6 @@ constexpr int kNormMaxThreads = 768;  // keeps ~170 VGPRs per lane for the norm 
 constexpr int kScoreP = 64;    // cache positions per score workgroup (one per lane)
 constexpr int kAttnHD = 256;   // head_dim served by the attention kernels
 
-// s = 0; s += v[i] for i = 0..n-1, each add rounded (v 16-byte aligned in
-// LDS).  Every lane of the calling wave runs the same chain on broadcast LDS
-// reads.  Two register batches alternate: one is added while the next one's
-// reads are in flight, with no copies between them, so the chain runs at the
-// latency of its dependent adds.
-__device__ float seq_sum(const float *v, int n)
-{
-    constexpr int B = 8;  // float4 per batch
-    const float4 *v4 = reinterpret_cast<const float4 *>(v);
-    float s = 0.0f;
-    const int nb = n / (4 * B);
-    auto add_batch = [&](const float4 (&c)[B]) {
-#pragma unroll
-        for (int k = 0; k < B; ++k) {
-            s += c[k].x;
-            s += c[k].y;
-            s += c[k].z;
-            s += c[k].w;
-        }
-    };
-    if (nb > 0) {
-        float4 a[B], b[B];
-#pragma unroll
-        for (int k = 0; k < B; ++k) a[k] = v4[k];
-        int i = 0;
-        for (; i + 2 <= nb; i += 2) {
-            // the batch after the last re-reads the last one (never added)
-            const int nbx = (i + 1) * B;
-#pragma unroll
-            for (int k = 0; k < B; ++k) b[k] = v4[nbx + k];
-            add_batch(a);
-            const int nba = (i + 2 < nb ? i + 2 : i + 1) * B;
-#pragma unroll
-            for (int k = 0; k < B; ++k) a[k] = v4[nba + k];
-            add_batch(b);
-        }
-        if (i < nb) add_batch(a);
-    }
-    for (int i = nb * 4 * B; i < n; ++i) s += v[i];
-    return s;
-}
-
 // out = rms_norm(x, w) (CudaDevice::rms_norm, cuda.rs:2102-2180; CPU
 // ops.rs:24-79), optionally also as a Q8_0 pack.  One workgroup.
 template <int CH>
@@ -833,7 +791,7 @@ __global__ __launch_bounds__(kScoreT) void attn_scores2_kernel(const float *__re
 // positions per 16-byte read, one tile behind the producers (one barrier per
 // tile, products double-buffered).
 // Writes out (nullable) and the Q8_0 pack of the n_heads*head_dim output
-// (nullable).  Dynamic LDS: capacity floats plus 4 (sv_lds).
+// (nullable).  Dynamic LDS: capacity floats (sv_lds).
 constexpr int kSVD = 32;  // dims per workgroup
 constexpr int kSVW = 8;   // waves: wave 0 adds; waves 1-3 and 5-7 produce; wave 4, which shares wave 0's SIMD, idles
 constexpr int kSVT = 96;  // positions per tile: 48 position pairs x 8 dim quads = one per producer thread
@@ -950,7 +908,7 @@ static_assert(kSVChunk <= mrml_xsum::kMaxPerThread * 64 * kSVW, "one block sum p
 __host__ __device__ constexpr bool sv_long(int capacity) { return capacity > kSVShortCap; }
 inline size_t sv_lds(int capacity)
 {
-    return sv_long(capacity) ? (size_t)kSVChunk * 5 + sizeof(mrml_xsum::Shared) : (size_t)capacity * sizeof(float) + 16;
+    return sv_long(capacity) ? (size_t)kSVChunk * 5 + sizeof(mrml_xsum::Shared) : (size_t)capacity * sizeof(float);
 }
 
 // VF: the V cache's format (0 f16, 1 Q8_0, 2 Q4_0; KvCacheFormat::cuda_code);
@@ -1061,15 +1019,25 @@ __global__ __launch_bounds__(64 * kSVW) void attn_softmax_v_kernel(const float *
         }
         sum = s;
     } else {
-        for (int p = tid; p < window; p += 64 * kSVW) e_s[p] = mrml_libm::expf_t(sc[p] - mx, fused_exp, exp_tab);
-        __syncthreads();
-        float *bcast = e_s + capacity;
-        if (wave == 0) {
-            const float s0 = seq_sum(e_s, window);
-            if (lane == 0) *bcast = s0;
+        // chunks of kSVE - 1 exps, the running sum prepended to each as its
+        // first term (0 + s = s is exact); one lane adding 3000 exps in order
+        // took 11 us, two chunks take 5
+        sum = 0.0f;
+        for (int c0 = 0; c0 < window; c0 += kSVE - 1) {
+            const int n = window - c0 < kSVE - 1 ? window - c0 : kSVE - 1;
+            float e[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int k = 4 * tid + i - 1;
+                e[i] = k < 0 ? sum : 0.0f;
+                if (k >= 0 && k < n) {
+                    e[i] = mrml_libm::expf_t(sc[c0 + k] - mx, fused_exp, exp_tab);
+                    e_s[c0 + k] = e[i];
+                }
+            }
+            sum = mrml_xsum::block_seq_sum_nonneg4(make_float4(e[0], e[1], e[2], e[3]), n + 1, *sum_x);
+            __syncthreads();  // the sum's LDS is reused
         }
-        __syncthreads();
-        sum = *bcast;
     }
     const SvWeights sw{sc, mx, sum > 0.0f ? 1.0f / sum : 1.0f, sum > 0.0f, fused_exp, exp_tab};
     if (!LONG && sum > 0.0f) {
