@@ -186,6 +186,121 @@ __global__ __launch_bounds__(64 * kRowsW) void attn_rows_scores_kernel(
     }
 }
 
+// Quantised K rows (KF 1: Q8_0, 2: Q4_0): dot_head is the block-ordered fold
+// s = s + (float)isum_b * (d_k * d_q) against the query's Q8_0 blocks
+// (kv_cache.rs:73-95).  The same tiling: the tile's blocks are re-laid in LDS
+// once (4-byte-aligned quants, f32 scales, odd row strides) and serve
+// kRowsQC chain rows a pass, `reps` passes, four a wave.  One row a workgroup
+// spent ten times its dots on that re-laying: 300 rows x 8 heads of 256 dims
+// over a window of 512 took 143 us.
+constexpr int kRowsQM = 4, kRowsQC = kRowsW * kRowsQM;  // chain rows a wave, a pass
+__host__ __device__ constexpr int rows_q_kstride(int kf, int nb) { return nb * (kf == 2 ? 4 : 8) + 1; }  // dwords
+inline size_t rows_q_lds(int kf, int nb)
+{
+    return 4 * ((size_t)kRowsP * (rows_q_kstride(kf, nb) + (nb | 1)) + 3 + (size_t)kRowsQC * nb * 10);
+}
+
+template <int KF>
+__global__ __launch_bounds__(64 * kRowsW) void attn_rows_scores_q_kernel(
+    const float *__restrict__ q, int q_stride, const uint8_t *__restrict__ k_cache, int n_past0, int nchains,
+    int n_heads, int n_kv_heads, int nb, float scale, int capacity, int wlimit, int t_lo, int reps,
+    float *__restrict__ scores)
+{
+    constexpr int M = kRowsQM, NT = 64 * kRowsW, BB = KF == 1 ? 34 : 18, QW = KF == 1 ? 8 : 4;
+    extern __shared__ __align__(16) uint32_t q_lds[];
+    const int HD = 32 * nb, KS = rows_q_kstride(KF, nb), DS = nb | 1, G = n_heads / n_kv_heads;
+    uint32_t *kq = q_lds;                                                   // [64][KS] quants
+    float *kd = reinterpret_cast<float *>(kq + kRowsP * KS);                // [64][DS] scales
+    uint32_t *qq = q_lds + ((kRowsP * (KS + DS) + 3) & ~3);                 // [kRowsQC][nb][8] query quants
+    float *qd = reinterpret_cast<float *>(qq + kRowsQC * nb * 8);           // [kRowsQC][nb] scales
+    int *qs = reinterpret_cast<int *>(qd + kRowsQC * nb);                   // [kRowsQC][nb] quant sums
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int T0 = t_lo + (int)blockIdx.x * kRowsP, kvh = blockIdx.y;
+    const int per = kRowsQC * reps, c0 = ((int)gridDim.z - 1 - (int)blockIdx.z) * per;
+    const int cl = (c0 + per < nchains ? c0 + per : nchains) - 1;  // the block's last chain row
+    int win0, start0;
+    attn_window(nullptr, n_past0 + c0 / G, wlimit, win0, start0);
+    const int pos_l = n_past0 + cl / G;
+    if (T0 > pos_l || start0 - T0 >= kRowsP) return;  // no row of the block has a position in this tile
+    {   // four threads a row, blocks tid % 4, + 4, ...
+        const int r = tid >> 2, t = T0 + r <= pos_l ? T0 + r : pos_l;
+        const uint8_t *krow = k_cache + (cache_row_of(t, capacity) * n_kv_heads + kvh) * ((size_t)nb * BB);
+        for (int b = tid & 3; b < nb; b += 4) {
+            const uint16_t *src = reinterpret_cast<const uint16_t *>(krow + b * BB);
+            uint32_t h[2 * QW];
+            const uint32_t d = src[0];
+#pragma unroll
+            for (int i = 0; i < 2 * QW; ++i) h[i] = src[1 + i];
+            kd[r * DS + b] = f16_bits_to_f32(d);
+#pragma unroll
+            for (int i = 0; i < QW; ++i) kq[r * KS + b * QW + i] = h[2 * i] | (h[2 * i + 1] << 16);
+        }
+    }
+    const int t = T0 + lane;
+    for (int rep = 0; rep < reps; ++rep) {
+        const int cp = c0 + rep * kRowsQC;
+        if (cp >= nchains) return;
+        __syncthreads();  // the tile is whole; the previous pass's queries are read
+        // eight lanes a block (every lane takes part in the quantiser's reductions)
+        for (int i0 = 0; i0 < kRowsQC * nb * 8; i0 += NT) {
+            const int i = i0 + tid, l = i & 7, cb = i >> 3, ci = cb / nb, b = cb - ci * nb;
+            const int c = cp + ci < nchains ? cp + ci : nchains - 1, z = c / G;
+            const float *src = q + (size_t)z * q_stride + (size_t)(kvh * G + c - z * G) * HD + 32 * b + 4 * l;
+            uint32_t dbits;
+            int sum;
+            const uint32_t v = q8_0_block8x4(make_float4(src[0], src[1], src[2], src[3]), dbits, sum);
+            if (ci >= kRowsQC) continue;  // (whole waves, past the pass's queries)
+            qq[i] = v;
+            if (l == 0) {
+                qd[cb] = f16_bits_to_f32(dbits);
+                qs[cb] = sum;
+            }
+        }
+        __syncthreads();
+        float acc[M];
+#pragma unroll
+        for (int m = 0; m < M; ++m) acc[m] = 0.0f;
+        for (int b = 0; b < nb; ++b) {
+            uint32_t kw[8];
+#pragma unroll
+            for (int i = 0; i < QW; ++i) {
+                const uint32_t w = kq[lane * KS + b * QW + i];
+                if constexpr (KF == 1) {
+                    kw[i] = w;
+                } else {  // low nibbles pair with values 0..15, high ones with 16..31
+                    kw[i] = w & 0x0F0F0F0Fu;
+                    kw[4 + i] = (w >> 4) & 0x0F0F0F0Fu;
+                }
+            }
+            const float d = kd[lane * DS + b];
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const int cb = (wave * M + m) * nb + b;
+                const u32x4 q0 = *reinterpret_cast<const u32x4 *>(&qq[cb * 8]);
+                const u32x4 q1 = *reinterpret_cast<const u32x4 *>(&qq[cb * 8 + 4]);
+                int isum = 0;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) isum = sdot4(kw[i], q0[i], isum);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) isum = sdot4(kw[4 + i], q1[i], isum);
+                if constexpr (KF == 2) isum -= 8 * qs[cb];  // (n - 8) . a = n . a - 8 * sum(a)
+                const float term = (float)isum * (d * qd[cb]);
+                acc[m] = acc[m] + term;
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            const int c = cp + wave * M + m, z = c / G;
+            if (c < nchains) {
+                int window, start;
+                attn_window(nullptr, n_past0 + z, wlimit, window, start);
+                if (t >= start && t < start + window)
+                    scores[((size_t)z * n_heads + kvh * G + c - z * G) * capacity + (t - start)] = acc[m] * scale;
+            }
+        }
+    }
+}
+
 // ---- softmax -----------------------------------------------------------------
 // Workgroup (head, row): the row's scores become its weights, in place.  Each
 // thread keeps four exps in registers for the register form of the exact
@@ -520,29 +635,43 @@ __global__ __launch_bounds__(256) void attn_rows_pv_kernel(const float *__restri
 
 }  // namespace
 
-// K rows are f16 (any head size that is a multiple of 32).
-int launch_attn_rows_scores(mrml_hip_ctx *ctx, const float *q, int q_stride, const uint16_t *k_cache, int n_past0,
-                            int rows, int n_heads, int n_kv_heads, int head_dim, float scale, int capacity, int wlimit,
+int launch_attn_rows_scores(mrml_hip_ctx *ctx, const float *q, int q_stride, const void *k_cache, int n_past0, int rows,
+                            int n_heads, int n_kv_heads, int head_dim, int k_fmt, float scale, int capacity, int wlimit,
                             float *scores)
 {
     const int G = n_heads / n_kv_heads, nchains = rows * G;
     // positions tiled absolutely from row 0's window start to the last row's position
     const int count0 = n_past0 + 1, t_lo = count0 > wlimit ? count0 - wlimit : 0, t_hi = n_past0 + rows - 1;
     const int tiles = (t_hi - t_lo) / kRowsP + 1;
+    const int64_t chain_tiles = (int64_t)tiles * n_kv_heads * nchains;
+    if (k_fmt != 0) {
+        // passes over a staged tile: as many as leave four workgroups a CU
+        const int reps = (int)std::min<int64_t>(8, std::max<int64_t>(1, chain_tiles / (kRowsQC * 1024)));
+        const int per = kRowsQC * reps;
+        const dim3 grid((unsigned)tiles, (unsigned)n_kv_heads, (unsigned)((nchains + per - 1) / per));
+#define ROWS_SCQ(KF)                                                                                               \
+    hipLaunchKernelGGL(attn_rows_scores_q_kernel<KF>, grid, dim3(64 * kRowsW), rows_q_lds(KF, head_dim / 32),       \
+                       ctx->stream, q, q_stride, (const uint8_t *)k_cache, n_past0, nchains, n_heads, n_kv_heads,   \
+                       head_dim / 32, scale, capacity, wlimit, t_lo, reps, scores)
+        if (k_fmt == 1) ROWS_SCQ(1);
+        else ROWS_SCQ(2);
+#undef ROWS_SCQ
+        return check_launch(ctx, "attn_rows_scores_q_kernel");
+    }
     // Chain rows a wave: four while that leaves two waves a SIMD, else two or
     // one (77 rows of 8 heads at 377 positions: 9.6 us with one, 11 with four).
     // Two sets of them a workgroup once the launch is many rounds of the chip
     // (512 rows behind 2048 positions: 10,240 workgroups, 7 us less; 512 rows
     // from the start: 2048, 2 us more).
-    const int64_t chain_tiles = (int64_t)tiles * n_kv_heads * nchains;
     const int M = chain_tiles >= 4 * 2048 ? 4 : (chain_tiles >= 2 * 2048 ? 2 : 1);
     const int reps = chain_tiles / (kRowsW * M) >= 8192 ? 2 : 1;
     const int per = kRowsW * M * reps;
     const dim3 grid((unsigned)tiles, (unsigned)n_kv_heads, (unsigned)((nchains + per - 1) / per));
     const size_t lds = (size_t)kRowsP * rows_k_stride(head_dim);
 #define ROWS_SC(M)                                                                                               \
-    hipLaunchKernelGGL(attn_rows_scores_kernel<M>, grid, dim3(64 * kRowsW), lds, ctx->stream, q, q_stride, k_cache, \
-                       n_past0, nchains, n_heads, n_kv_heads, head_dim, scale, capacity, wlimit, t_lo, reps, scores)
+    hipLaunchKernelGGL(attn_rows_scores_kernel<M>, grid, dim3(64 * kRowsW), lds, ctx->stream, q, q_stride,          \
+                       (const uint16_t *)k_cache, n_past0, nchains, n_heads, n_kv_heads, head_dim, scale, capacity, \
+                       wlimit, t_lo, reps, scores)
     if (M == 4) ROWS_SC(4);
     else if (M == 2) ROWS_SC(2);
     else ROWS_SC(1);

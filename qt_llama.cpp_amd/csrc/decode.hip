@@ -441,7 +441,7 @@ __global__ __launch_bounds__(64) void kv_append_any_kernel(const float *__restri
 // order; Q8_0 / Q4_0: the block-ordered fold s = s + (float)isum_b * (d_k *
 // d_q) over the head's blocks against quantize_f32_to_q8_0(q_h) (formed
 // here, per head, with the reference quantiser).  Workgroup (tile of 64
-// positions, kv head, query row): lane p owns position p0 + p and wave w
+// positions, kv head): lane p owns position p0 + p and wave w
 // the heads w, w + 4, ... of the group; the K tile is staged through LDS in
 // passes of 128 dims (f16 rows as they are; quantised blocks re-laid as
 // 4-byte-aligned quants plus f32 scales), every chain carried across passes
@@ -467,13 +467,9 @@ __global__ __launch_bounds__(kAnyT) void attn_scores_any_kernel(const float *__r
                                                                 const uint8_t *__restrict__ k_cache,
                                                                 const int32_t *__restrict__ d_pos, int n_past_arg,
                                                                 int n_heads, int n_kv_heads, int head_dim, float scale,
-                                                                int capacity, int wlimit, float *__restrict__ scores,
-                                                                int q_stride)
+                                                                int capacity, int wlimit, float *__restrict__ scores)
 {
     extern __shared__ __align__(16) uint8_t lds_any[];
-    q += (size_t)blockIdx.z * q_stride;
-    scores += (size_t)blockIdx.z * n_heads * capacity;
-    n_past_arg += (int)blockIdx.z;
     int window, start;
     attn_window(d_pos, n_past_arg, wlimit, window, start);
     const int p0 = blockIdx.x * kAnyP;
@@ -1634,19 +1630,20 @@ bool attn_tuned(int n_heads, int n_kv_heads, int head_dim, int k_fmt, int v_fmt)
     return head_dim == kAttnHD && k_fmt == 0 && v_fmt == 0 && n_kv_heads > 0 && n_heads / n_kv_heads <= 8;
 }
 
-// Scores over K rows of format k_fmt, one workgroup a (64 positions, kv head, row).
-static int launch_any_scores(mrml_hip_ctx *ctx, const float *q, int q_stride, const void *k_cache, const int32_t *d_pos,
-                             int n_past0, int rows, int n_heads, int n_kv_heads, int head_dim, int k_fmt, float scale,
-                             int capacity, int wlimit, float *scores)
+int launch_attn_any(mrml_hip_ctx *ctx, const float *q, const void *k_cache, const void *v_cache, float *out, void *pack,
+                    const int32_t *d_pos, int n_past, int n_heads, int n_kv_heads, int head_dim, int k_fmt, int v_fmt,
+                    float scale, int capacity, void *scratch, int sliding_window)
 {
-    // score tiles up to the widest row window (every tile when the position is on the device)
-    const int span = d_pos ? wlimit : std::min(wlimit, n_past0 + rows);
-    const dim3 sgrid((span + kAnyP - 1) / kAnyP, n_kv_heads, rows);
+    float *scores = reinterpret_cast<float *>(scratch);
+    const int wlimit = attn_window_limit(capacity, sliding_window);
+    // score tiles up to the window (every tile when the position is on the device)
+    const int span = d_pos ? wlimit : std::min(wlimit, n_past + 1);
+    const dim3 sgrid((span + kAnyP - 1) / kAnyP, n_kv_heads);
     const size_t lds = attn_any_scores_lds(k_fmt, n_heads / n_kv_heads, head_dim);
     const uint8_t *kc = reinterpret_cast<const uint8_t *>(k_cache);
 #define SC_LAUNCH(KF)                                                                                             \
-    hipLaunchKernelGGL(attn_scores_any_kernel<KF>, sgrid, dim3(kAnyT), lds, ctx->stream, q, kc, d_pos, n_past0,  \
-                       n_heads, n_kv_heads, head_dim, scale, capacity, wlimit, scores, q_stride)
+    hipLaunchKernelGGL(attn_scores_any_kernel<KF>, sgrid, dim3(kAnyT), lds, ctx->stream, q, kc, d_pos, n_past,    \
+                       n_heads, n_kv_heads, head_dim, scale, capacity, wlimit, scores)
     if (k_fmt == 1)
         SC_LAUNCH(1);
     else if (k_fmt == 2)
@@ -1654,18 +1651,7 @@ static int launch_any_scores(mrml_hip_ctx *ctx, const float *q, int q_stride, co
     else
         SC_LAUNCH(0);
 #undef SC_LAUNCH
-    return check_launch(ctx, "attn_scores_any_kernel");
-}
-
-int launch_attn_any(mrml_hip_ctx *ctx, const float *q, const void *k_cache, const void *v_cache, float *out, void *pack,
-                    const int32_t *d_pos, int n_past, int n_heads, int n_kv_heads, int head_dim, int k_fmt, int v_fmt,
-                    float scale, int capacity, void *scratch, int sliding_window)
-{
-    float *scores = reinterpret_cast<float *>(scratch);
-    const int wlimit = attn_window_limit(capacity, sliding_window);
-    if (int rc = launch_any_scores(ctx, q, 0, k_cache, d_pos, n_past, 1, n_heads, n_kv_heads, head_dim, k_fmt, scale,
-                                   capacity, wlimit, scores))
-        return rc;
+    if (int rc = check_launch(ctx, "attn_scores_any_kernel")) return rc;
     return launch_softmax_v(ctx, scores, v_cache, out, pack, d_pos, n_past, n_heads, n_kv_heads, capacity, wlimit, 1,
                             head_dim, v_fmt);
 }
@@ -1682,11 +1668,8 @@ int launch_attn_rows(mrml_hip_ctx *ctx, const float *q, int q_stride, const void
 {
     float *scores = reinterpret_cast<float *>(scratch);
     const int wlimit = attn_window_limit(capacity, sliding_window), span = std::min(wlimit, n_past0 + rows);
-    if (int rc = k_fmt == 0
-                     ? launch_attn_rows_scores(ctx, q, q_stride, (const uint16_t *)k_cache, n_past0, rows, n_heads,
-                                               n_kv_heads, head_dim, scale, capacity, wlimit, scores)
-                     : launch_any_scores(ctx, q, q_stride, k_cache, nullptr, n_past0, rows, n_heads, n_kv_heads,
-                                         head_dim, k_fmt, scale, capacity, wlimit, scores))
+    if (int rc = launch_attn_rows_scores(ctx, q, q_stride, k_cache, n_past0, rows, n_heads, n_kv_heads, head_dim, k_fmt,
+                                         scale, capacity, wlimit, scores))
         return rc;
     // The decode form's workgroup adds 32 dims of one row at 4.7 ns a
     // position, the rows form's waves need company for that: while the decode

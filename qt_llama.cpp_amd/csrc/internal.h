@@ -217,10 +217,10 @@ bool attn_rope_ok(int n_heads, int n_kv_heads);
 int launch_attn_rows(mrml_hip_ctx *ctx, const float *q, int q_stride, const void *k_cache, const void *v_cache,
                      float *out, int n_past0, int rows, int n_heads, int n_kv_heads, int head_dim, int k_fmt, int v_fmt,
                      float scale, int capacity, void *scratch, int sliding_window);
-// Its parts in attn_rows.hip: scores over f16 K rows; softmax and weighted sum
+// Its parts in attn_rows.hip: scores; softmax and weighted sum
 // (caches that attn_rows_v_ok says a buffer descriptor reaches).
-int launch_attn_rows_scores(mrml_hip_ctx *ctx, const float *q, int q_stride, const uint16_t *k_cache, int n_past0,
-                            int rows, int n_heads, int n_kv_heads, int head_dim, float scale, int capacity, int wlimit,
+int launch_attn_rows_scores(mrml_hip_ctx *ctx, const float *q, int q_stride, const void *k_cache, int n_past0, int rows,
+                            int n_heads, int n_kv_heads, int head_dim, int k_fmt, float scale, int capacity, int wlimit,
                             float *scores);
 bool attn_rows_v_ok(int n_kv_heads, int head_dim, int v_fmt, int capacity);
 int launch_attn_rows_softmax_v(mrml_hip_ctx *ctx, float *scores, const void *v_cache, float *out, int n_past0, int rows,
