@@ -453,8 +453,8 @@ int mrml_hip_add(mrml_hip_ctx *ctx, const float *d_a, const float *d_b, float *d
  * min(n_past+1, capacity) cache rows, kv head h / (n_heads / n_kv_heads),
  * in the CPU path's operation order (sequential dots, softmax sum and
  * weighted sum; the host C library's expf).  head_dim a multiple of 32 up
- * to 512, groups of at most 16, capacity at most 2^20: past 6144 the
- * window's exps are summed in LDS-staged chunks, each chunk's exact
+ * to 512, groups of at most 16, capacity at most 2^20: past 10240
+ * positions the window's exps are summed in LDS-staged chunks, each chunk's exact
  * sequential sum continuing the running sum (the same bits; the reference
  * streams such windows through its online-softmax kernel,
  * kernels.rs:1463-1561).  d_out (f32) and d_pack (Q8_0 pack of the

@@ -787,7 +787,7 @@ __global__ __launch_bounds__(kScoreT) void attn_scores2_kernel(const float *__re
 // positions per 16-byte read, one tile behind the producers (one barrier per
 // tile, products double-buffered).
 // Writes out (nullable) and the Q8_0 pack of the n_heads*head_dim output
-// (nullable).  Dynamic LDS: capacity floats (sv_lds).
+// (nullable).  Dynamic LDS: a float a position of the widest window (sv_lds).
 constexpr int kSVD = 32;  // dims per workgroup
 constexpr int kSVW = 8;   // waves: wave 0 adds; waves 1-3 and 5-7 produce; wave 4, which shares wave 0's SIMD, idles
 constexpr int kSVT = 96;  // positions per tile: 48 position pairs x 8 dim quads = one per producer thread
@@ -890,21 +890,29 @@ __device__ __forceinline__ void sv_products(const u32x2 (&r)[kSVR], const float 
         *reinterpret_cast<float2 *>(&prod[4 * dq + d][kSVR * tq]) = make_float2(pv[d][0], pv[d][1]);
 }
 
-// LONG (capacities past kSVShortCap): the window's weights do not fit in
-// LDS.  The sum then runs over chunks of kSVChunk - 1 exps staged in LDS,
+// LONG (windows past kSVShort positions): the weights are not kept in LDS,
+// and a producer forms one again for every dim quad of every slice.  The sum runs over chunks of kSVChunk - 1 exps staged in LDS,
 // each chunk's exact sequential sum started from the running sum (prepended
 // as the chunk's first term: s = 0 + s_prev is exact, so the chunked sums
 // equal the one sequential loop), and the producers form their weights from
 // the global scores.  Dynamic LDS: kSVChunk floats, kSVChunk flag bytes and
 // the block sum's Shared.
-constexpr int kSVShortCap = 6144;  // the LDS form keeps capacity floats of weights
+//
+// The line lies on the widest window of the launch, not on the cache's
+// capacity, and where the weights take as much LDS as LONG's chunk and flags:
+// up to there the LDS form costs no resident workgroup.  Attention in caches
+// of 8192 positions, LONG / LDS form: 5310 positions, 4 heads of 64 dims over
+// Q4_0 rows 65.6 / 41.9 us; 2774, 8 heads of 128 over f16 36.8 / 25.4; a window
+// of 1024, 16 heads of 128 over Q8_0/Q4_0 23.2 / 19.5.
+constexpr int kSVShort = 10240;  // positions: 40 KiB of weights
 constexpr int kSVChunk = 8192;     // LONG: terms per exact block sum (16 per thread)
 static_assert(kSVChunk <= mrml_xsum::kMaxPerThread * 64 * kSVW, "one block sum per chunk");
 
-__host__ __device__ constexpr bool sv_long(int capacity) { return capacity > kSVShortCap; }
-inline size_t sv_lds(int capacity)
+__host__ __device__ constexpr bool sv_long(int span) { return span > kSVShort; }
+inline size_t sv_lds(int span)  // (weights are read in pairs)
 {
-    return sv_long(capacity) ? (size_t)kSVChunk * 5 + sizeof(mrml_xsum::Shared) : (size_t)capacity * sizeof(float);
+    return sv_long(span) ? (size_t)kSVChunk * 5 + sizeof(mrml_xsum::Shared)
+                         : ((size_t)span + 3) / 4 * 4 * sizeof(float);
 }
 
 // VF: the V cache's format (0 f16, 1 Q8_0, 2 Q4_0; KvCacheFormat::cuda_code);
@@ -1275,7 +1283,7 @@ __global__ __launch_bounds__(kAttnHD) void attn_combine_kernel(const float *__re
                                                                int capacity, int wlimit, int max_tiles, int n_heads,
                                                                float *__restrict__ out, uint8_t *__restrict__ pack)
 {
-    constexpr int HD = kAttnHD, kMaxTiles = (kSVShortCap + kSplitP - 1) / kSplitP;
+    constexpr int HD = kAttnHD, kMaxTiles = 192;  // 6144 positions; more take the loop over tiles
     __shared__ float m_s[kMaxTiles], w_s[kMaxTiles], l_s[kMaxTiles];
     __shared__ float red[HD / 64];
     static_assert(kMaxTiles <= HD, "one tile's (m, l) per thread");
@@ -1554,8 +1562,14 @@ int attn_max_capacity() { return 1 << 20; }
 
 size_t attn_scratch_bytes(int n_heads, int capacity) { return (size_t)n_heads * capacity * sizeof(float); }
 
+// The widest window of `rows` rows from position n_past on; any, if the position is on the device.
+static int attn_span(const int32_t *d_pos, int n_past, int rows, int wlimit)
+{
+    return d_pos ? wlimit : (int)std::min<int64_t>(wlimit, (int64_t)n_past + rows);
+}
+
 // Softmax and weighted values of `rows` query rows (grid z), the LDS or the
-// LONG form by capacity, V rows in format v_fmt.
+// LONG form by their widest window, V rows in format v_fmt.
 static int launch_softmax_v(mrml_hip_ctx *ctx, const float *scores, const void *v_cache, float *out, void *pack,
                             const int32_t *d_pos, int n_past, int n_heads, int n_kv_heads, int capacity, int wlimit,
                             int rows = 1, int head_dim = kAttnHD, int v_fmt = 0)
@@ -1564,9 +1578,10 @@ static int launch_softmax_v(mrml_hip_ctx *ctx, const float *scores, const void *
     const uint8_t *v = reinterpret_cast<const uint8_t *>(v_cache);
     const int fe = (int)host_expf_fused();
 #define SV_LAUNCH(LONG, VF)                                                                                          \
-    hipLaunchKernelGGL((attn_softmax_v_kernel<LONG, VF>), grid, block, sv_lds(capacity), ctx->stream, scores, v,   \
+    hipLaunchKernelGGL((attn_softmax_v_kernel<LONG, VF>), grid, block, sv_lds(span), ctx->stream, scores, v,       \
                        d_pos, n_past, n_heads, n_kv_heads, head_dim, capacity, wlimit, fe, out, (uint8_t *)pack)
-    const bool lg = sv_long(capacity);
+    const int span = attn_span(d_pos, n_past, rows, wlimit);
+    const bool lg = sv_long(span);
     if (v_fmt == 1) {
         if (lg) SV_LAUNCH(true, 1); else SV_LAUNCH(false, 1);
     } else if (v_fmt == 2) {
@@ -1583,8 +1598,8 @@ int launch_attn_decode_f16(mrml_hip_ctx *ctx, const float *q, const uint16_t *k_
                            float scale, int capacity, void *scratch, int sliding_window)
 {
     float *scores = reinterpret_cast<float *>(scratch);
-    const dim3 sgrid((capacity + kScoreP - 1) / kScoreP, n_kv_heads);
     const int wlimit = attn_window_limit(capacity, sliding_window);
+    const dim3 sgrid((attn_span(d_pos, n_past, 1, wlimit) + kScoreP - 1) / kScoreP, n_kv_heads);
     if (n_heads / n_kv_heads <= 4) {
         hipLaunchKernelGGL(attn_scores2_kernel<false>, sgrid, dim3(kScoreT), 0, ctx->stream, q,
                            const_cast<uint16_t *>(k_cache), (uint16_t *)nullptr, d_pos, n_past, n_heads, n_kv_heads,
@@ -1637,8 +1652,7 @@ int launch_attn_any(mrml_hip_ctx *ctx, const float *q, const void *k_cache, cons
     float *scores = reinterpret_cast<float *>(scratch);
     const int wlimit = attn_window_limit(capacity, sliding_window);
     // score tiles up to the window (every tile when the position is on the device)
-    const int span = d_pos ? wlimit : std::min(wlimit, n_past + 1);
-    const dim3 sgrid((span + kAnyP - 1) / kAnyP, n_kv_heads);
+    const dim3 sgrid((attn_span(d_pos, n_past, 1, wlimit) + kAnyP - 1) / kAnyP, n_kv_heads);
     const size_t lds = attn_any_scores_lds(k_fmt, n_heads / n_kv_heads, head_dim);
     const uint8_t *kc = reinterpret_cast<const uint8_t *>(k_cache);
 #define SC_LAUNCH(KF)                                                                                             \

@@ -93,6 +93,31 @@ def test_attention_any_bit_exact(backend, dev, orc, nh, nkv, hd, kf, vf, cap, sw
         qb.close()
 
 
+# Windows on both sides of the line (10240 positions) between the weights in
+# LDS and the long form, odd ones and chunk ends among them, in larger caches;
+# sliding windows far below the capacity.
+@pytest.mark.parametrize("nh,nkv,hd,kf,vf,cap,sw,n_pasts", [
+    (8, 4, 256, 0, 0, 16384, None, [2048, 8190, 10238, 10239, 10240]),
+    (16, 2, 128, 1, 2, 16384, 1024, [700, 15000]),
+    (4, 2, 64, 2, 1, 16384, 10239, [10300]),
+    (2, 1, 32, 0, 0, 12000, 10241, [10239, 12100]),
+])
+def test_attention_window_line_bit_exact(backend, dev, orc, nh, nkv, hd, kf, vf, cap, sw, n_pasts):
+    rng = np.random.default_rng(8123 + hd)
+    kc, vc = (cache_bytes(orc, rng.standard_normal((cap, nkv * hd), dtype=np.float32), f) for f in (kf, vf))
+    kb, vb = upload_cache(backend, dev, kc), upload_cache(backend, dev, vc)
+    out = backend.HipBuffer.alloc(dev, nh * hd)
+    q = rng.standard_normal(nh * hd, dtype=np.float32)
+    qb = backend.HipBuffer.from_host(dev, q)
+    scale = float(np.float32(1.0 / np.sqrt(hd)))
+    for n_past in n_pasts:
+        print(f"\n[attention line] hd {hd} n_past {n_past}", flush=True)
+        dev.attention_causal_ref(qb, kb, vb, out, n_past, nh, nkv, hd, scale, sw, cap, kf, vf)
+        dev.sync()
+        ref = oracle_rows(orc, q, kc, vc, n_past, sw, cap, nh, nkv, hd, scale, kf, vf)
+        assert_bits(out.numpy(), ref, f"n_past {n_past}")
+
+
 def test_attention_reference_head_dim_64_case(backend, dev, orc):
     """ops_test.rs:375-449 (test_cuda_causal_attention_matches_cpu): 4 query
     and 2 kv heads of 64, 8 tokens, sliding window 4, capacity 8, caches of
