@@ -340,16 +340,38 @@ __device__ __forceinline__ T block_max(T v, T *red)
     return m;
 }
 
+// How many of vals[0..n) (LDS; P * 8 entries at a time are read, so the array
+// is that much rounded up) pass, over the P adjacent threads of a value, each
+// taking every P-th.  A count is bound by the LDS round trip of its reads, so
+// eight are in flight and the values have P threads each.  (With the ordered
+// sums of the draw over registers, not LDS, and no second selection where few
+// candidates are left: Q4_K product and top-40 draw over 256000 ids 93.8 ->
+// 78.1 us, of which the product is 50.)
+template <int P, typename T, typename F>
+__device__ __forceinline__ int count_if(const T *vals, int n, F pass)
+{
+    int c = 0;
+    for (int u0 = (int)threadIdx.x % P; u0 < n; u0 += 8 * P) {
+        T x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = vals[u0 + i * P];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) c += u0 + i * P < n && pass(x[i]) ? 1 : 0;
+    }
+#pragma unroll
+    for (int off = 1; off < P; off <<= 1) c += __shfl_xor(c, off, 64);
+    return c;
+}
+
 // The k-th largest of vals[0..n) (LDS), counted with multiplicity: the
 // largest v with at least k values >= v; `none` when n < k.  Every thread.
-template <typename T>
+template <int P, typename T>
 __device__ __forceinline__ T kth_largest(const T *vals, int n, int k, T none, T *red)
 {
     T best = none;
-    for (int t = threadIdx.x; t < n; t += blockDim.x) {
+    for (int t = (int)threadIdx.x / P; t < n; t += (int)blockDim.x / P) {
         const T v = vals[t];
-        int c = 0;
-        for (int u = 0; u < n; ++u) c += vals[u] >= v ? 1 : 0;
+        const int c = count_if<P>(vals, n, [v](T x) { return x >= v; });
         if (c >= k && v > best) best = v;
     }
     return block_max(best, red);
@@ -358,13 +380,13 @@ __device__ __forceinline__ T kth_largest(const T *vals, int n, int k, T none, T 
 // top[0..k) = the k largest of the n_surv distinct non-zero keys in surv
 // (LDS), descending, then zeros: each key's rank is the number of larger
 // ones.  Ends with a barrier.
+template <int P>
 __device__ __forceinline__ void rank_survivors(const uint64_t *surv, int n_surv, int k, uint64_t *top)
 {
-    for (int s = threadIdx.x; s < n_surv; s += blockDim.x) {
+    for (int s = (int)threadIdx.x / P; s < n_surv; s += (int)blockDim.x / P) {
         const uint64_t x = surv[s];
-        int r = 0;
-        for (int u = 0; u < n_surv && r < k; ++u) r += surv[u] > x ? 1 : 0;  // k or more: placed nowhere
-        if (r < k) top[r] = x;
+        const int r = count_if<P>(surv, n_surv, [x](uint64_t y) { return y > x; });
+        if (r < k && (int)threadIdx.x % P == 0) top[r] = x;  // k or more: placed nowhere
     }
     for (int i = n_surv + (int)threadIdx.x; i < k; i += blockDim.x) top[i] = 0;
     __syncthreads();
@@ -471,7 +493,7 @@ __device__ __forceinline__ void merge_lists(const uint64_t *__restrict__ lists, 
     }
     m.heads[t] = t < n_lists ? lists[(size_t)t * k] : 0;
     __syncthreads();
-    uint64_t L = kth_largest(m.heads, n_lists, k, (uint64_t)0, m.red);
+    uint64_t L = kth_largest<8>(m.heads, n_lists, k, (uint64_t)0, m.red);
     L = L ? L : 1;
     // the lists with a head >= L (at most k: the heads are distinct keys or 0)
     if (t < n_lists && m.heads[t] >= L) {
@@ -485,38 +507,44 @@ __device__ __forceinline__ void merge_lists(const uint64_t *__restrict__ lists, 
     // length is the largest place that passes, plus one
     const int ns = m.n_seg, npairs = ns * k;
     constexpr int kPairs = kTopKMax * kTopKMax / kSelectThreads;
+    // q / k as a product: exact for q < 2^12, k <= 2^6 (the reciprocal's excess is below k / 2^20)
+    const uint32_t rk = ((1u << 20) + (uint32_t)k - 1) / (uint32_t)k;
+    auto seg_of = [rk](int q) { return (int)(((uint32_t)q * rk) >> 20); };
     static_assert(kPairs * kSelectThreads == kTopKMax * kTopKMax, "whole pairs per thread");
     uint64_t pk[kPairs];
 #pragma unroll
     for (int i = 0; i < kPairs; ++i) {
         const int q = t + i * kSelectThreads;
-        pk[i] = q < npairs ? lists[(size_t)m.seg_list[q / k] * k + q % k] : 0;
+        pk[i] = q < npairs ? lists[(size_t)m.seg_list[seg_of(q)] * k + (q - seg_of(q) * k)] : 0;
     }
 #pragma unroll
     for (int i = 0; i < kPairs; ++i) {
         const int q = t + i * kSelectThreads;
-        if (q < npairs && pk[i] >= L) atomicMax(&m.seg_len[q / k], q % k + 1);
+        if (q < npairs && pk[i] >= L) atomicMax(&m.seg_len[seg_of(q)], q - seg_of(q) * k + 1);
     }
     __syncthreads();
-    if (t == 0) {
-        int off = 0;
-        for (int sg = 0; sg < ns; ++sg) {
-            m.seg_off[sg] = off;
-            off += m.seg_len[sg];
+    if (t < 64) {  // at most k <= 64 segments: offsets by a wave scan
+        const int len = t < ns ? m.seg_len[t] : 0;
+        int end = len;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int o = __shfl_up(end, off, 64);
+            end += t >= off ? o : 0;
         }
-        m.n_surv = off;
+        if (t < ns) m.seg_off[t] = end - len;
+        if (t == 63) m.n_surv = end;
     }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < kPairs; ++i) {
-        const int q = t + i * kSelectThreads, sg = q / k, j = q % k;
+        const int q = t + i * kSelectThreads, sg = seg_of(q), j = q - sg * k;
         if (q < npairs && j < m.seg_len[sg]) {
             m.surv[m.seg_off[sg] + j] = pk[i];
             m.surv_seg[m.seg_off[sg] + j] = (uint8_t)sg;
         }
     }
     __syncthreads();
-    if (m.n_surv <= 4 * kTopKMax) rank_survivors(m.surv, m.n_surv, k, top);
+    if (m.n_surv <= 4 * kTopKMax) rank_survivors<16>(m.surv, m.n_surv, k, top);
     else rank_segments(m.surv, m.surv_seg, m.n_surv, m.seg_off, m.seg_len, m.n_seg, k, top);
 }
 
@@ -560,7 +588,7 @@ __global__ __launch_bounds__(kVocabThreads) void vocab_topk_partial_kernel(Vocab
     constexpr int N = kVocabPerThread;
     __shared__ int32_t rec[kRecentMax];
     __shared__ int n_rec, n_surv, n_cand;
-    __shared__ float fred[kVocabThreads / 64], fvals[kVocabThreads];
+    __shared__ float fred[kVocabThreads / 64], fvals[kVocabThreads / 2];
     __shared__ float c_val[kVocabPart];
     __shared__ uint16_t c_meta[kVocabPart];
     __shared__ uint64_t c_key[kVocabPart];
@@ -598,6 +626,7 @@ __global__ __launch_bounds__(kVocabThreads) void vocab_topk_partial_kernel(Vocab
             n_cand = 0;
         }
     }
+    if (threadIdx.x < kTopKMax) top[threadIdx.x] = 0;
     __syncthreads();
     const int nr = n_rec;
     // scores: exact for the device path; for the CPU path an interval
@@ -628,15 +657,18 @@ __global__ __launch_bounds__(kVocabThreads) void vocab_topk_partial_kernel(Vocab
         mlo = lo[i] > mlo ? lo[i] : mlo;
     }
     // T: a lower bound of the partition's k-th best score (the k-th largest
-    // per-thread best lower end); only candidates with hi >= T can place.
-    // They are compacted (element, value, penalty) for one exact pass.
+    // best lower end of a thread pair); only candidates with hi >= T can place.
+    // They are compacted (element, value, penalty) for one exact pass.  Pairs
+    // halve the values to count against and let through 47 candidates at
+    // k = 40 where single threads let through 43.
     float T;
     if (k == 1) {
         T = block_max(mlo, fred);
     } else {
-        fvals[threadIdx.x] = mlo;
+        const float other = __shfl_xor(mlo, 1, 64), both = other > mlo ? other : mlo;
+        if ((threadIdx.x & 1) == 0) fvals[threadIdx.x >> 1] = both;
         __syncthreads();
-        T = kth_largest(fvals, kVocabThreads, k, -INFINITY, fred);
+        T = kth_largest<2>(fvals, kVocabThreads / 2, k, -INFINITY, fred);
     }
 #pragma unroll
     for (int i = 0; i < N; ++i)
@@ -664,7 +696,9 @@ __global__ __launch_bounds__(kVocabThreads) void vocab_topk_partial_kernel(Vocab
         const int s = i * kVocabThreads + (int)threadIdx.x;
         keys[i] = s < nc ? c_key[s] : 0;
     }
-    if (k == 1) {
+    if (k > 1 && nc <= kVocabThreads) {  // few candidates (the usual case): their ranks at once
+        rank_survivors<4>(c_key, nc, k, top);
+    } else if (k == 1) {
         uint64_t b = 0;
 #pragma unroll
         for (int i = 0; i < N; ++i) b = keys[i] > b ? keys[i] : b;
@@ -677,13 +711,13 @@ __global__ __launch_bounds__(kVocabThreads) void vocab_topk_partial_kernel(Vocab
         sort_desc(keys);
         heads[threadIdx.x] = keys[0];
         __syncthreads();
-        uint64_t L = kth_largest(heads, kVocabThreads, k, (uint64_t)0, kred);
+        uint64_t L = kth_largest<1>(heads, kVocabThreads, k, (uint64_t)0, kred);
         L = L ? L : 1;
 #pragma unroll
         for (int i = 0; i < N; ++i)
             if (keys[i] >= L) surv[atomicAdd(&n_surv, 1)] = keys[i];
         __syncthreads();
-        rank_survivors(surv, n_surv, k, top);
+        rank_survivors<4>(surv, n_surv, k, top);
     }
     for (int r = threadIdx.x; r < k; r += blockDim.x) {
         const uint64_t key = top[r];
@@ -726,48 +760,46 @@ __global__ __launch_bounds__(kSelectThreads) void vocab_select_kernel(
 {
     __shared__ MergeShared ms;
     __shared__ uint64_t top[kTopKMax];
-    __shared__ float probs[kTopKMax], quot[kTopKMax];
     merge_lists(part, n_part, k, top, ms);
     const int t = threadIdx.x;
-    int n = 0;
-    for (int i = 0; i < k; ++i) n += top[i] != 0 ? 1 : 0;  // the candidates lead, zeros follow
-    // the CPU path's state.pos: the position after the token just processed
-    const unsigned long long pos = state ? (unsigned long long)state[1] + 1ull : pos_arg;
-    const bool draw = n > 0 && temperature > 0.0f;
-    if (draw) {
-        const float s0 = key_score(top[0]);
+    if (t >= 64) return;
+    // wave 0, lane t = candidate t (they lead, zeros follow); the reference's
+    // ordered sums run over the lanes' registers
+    const uint64_t key = t < k ? top[t] : 0;
+    const int n = (int)__popcll(__ballot(key != 0));
+    const int id = key ? key_id(key) : -1;
+    const float score = key ? key_score(key) : -INFINITY;
+    if (t < k) {
+        if (out_scores) out_scores[t] = score;
+        if (out_ids) out_ids[t] = id;
+    }
+    auto lane_f32 = [](float v, int l) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+    };
+    int token = n ? __builtin_amdgcn_readlane(id, 0) : 506;
+    if (n > 0 && temperature > 0.0f) {
+        // the CPU path's state.pos: the position after the token just processed
+        const unsigned long long pos = state ? (unsigned long long)state[1] + 1ull : pos_arg;
+        const float s0 = lane_f32(score, 0);
         const float temp = temperature > 0.1f ? temperature : 0.1f;
-        if (t < n) probs[t] = mrml_libm::expf((key_score(top[t]) - s0) / temp, expf_fused != 0);
-        __syncthreads();
-        if (t < n) {
-            float sum_exp = 0.0f;
-            for (int i = 0; i < n; ++i) sum_exp += probs[i];
-            quot[t] = probs[t] / sum_exp;
+        const float prob = t < n ? mrml_libm::expf((score - s0) / temp, expf_fused != 0) : 0.0f;
+        float sum_exp = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kTopKMax; ++i) sum_exp += lane_f32(prob, i);  // (+ 0 past the candidates)
+        if (sum_exp > 0.0f) {
+            const float quot = prob / sum_exp;
+            const float rng = (float)((pos * 6364136223846793005ull + 1ull) >> 33) / (float)0xffffffffu;
+            float acc = 0.0f, mine = 0.0f;  // mine: the sum up to this lane's candidate
+#pragma unroll
+            for (int i = 0; i < kTopKMax; ++i) {
+                acc += lane_f32(quot, i);
+                mine = t == i ? acc : mine;
+            }
+            const uint64_t hit = __ballot(t < n && rng <= mine);
+            if (hit) token = __builtin_amdgcn_readlane(id, __builtin_ctzll(hit));
         }
-        __syncthreads();
     }
     if (t != 0) return;
-    if (out_scores || out_ids)
-        for (int i = 0; i < k; ++i) {
-            if (out_scores) out_scores[i] = i < n ? key_score(top[i]) : -INFINITY;
-            if (out_ids) out_ids[i] = i < n ? key_id(top[i]) : -1;
-        }
-    int token = n ? key_id(top[0]) : 506;
-    if (draw) {
-        float sum_exp = 0.0f;
-        for (int i = 0; i < n; ++i) sum_exp += probs[i];
-        if (sum_exp > 0.0f) {
-            const float rng = (float)((pos * 6364136223846793005ull + 1ull) >> 33) / (float)0xffffffffu;
-            float acc = 0.0f;
-            for (int i = 0; i < n; ++i) {
-                acc += quot[i];
-                if (rng <= acc) {
-                    token = key_id(top[i]);
-                    break;
-                }
-            }
-        }
-    }
     if (out_token) *out_token = token;
     if (state) {
         const int cur = state[1];

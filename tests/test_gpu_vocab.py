@@ -80,6 +80,32 @@ def test_vocab_select_edges(backend, dev, orc):
                              f"vocab={vocab} scoring={scoring} t={temp}")
 
 
+# A partition whose candidates near the k-th best fit a thread each, and one
+# where they do not (equal and nearly equal logits); list counts at the edges
+# of the merge's counting groups; a whole short list in every partition (the
+# merge's segment form: more than 256 survivors); the largest list count.
+@pytest.mark.parametrize("vocab", [255, 2048, 2049, 8 * 2048, 64 * 2048 + 1, 128 * 2048, 129 * 2048 + 5, 1024 * 2048])
+@pytest.mark.parametrize("shape", ["spread", "flat", "near", "few", "blocks"])
+def test_vocab_select_forms(backend, dev, orc, vocab, shape):
+    rng = np.random.default_rng(vocab + len(shape))
+    lg = (rng.standard_normal(vocab) * 6.0).astype(np.float32)
+    valid = np.ones(vocab, np.uint8)
+    if shape == "flat":
+        lg[:] = 2.5
+    elif shape == "near":  # every interval of the cheap scoring overlaps
+        lg = (1.0 + rng.random(vocab) * 1e-3).astype(np.float32)
+    elif shape == "few":
+        valid = (rng.random(vocab) < 1e-3).astype(np.uint8)
+    elif shape == "blocks":  # partitions in descending order: one list holds every survivor
+        lg = np.sort(lg)[::-1].copy()
+    recent = rng.integers(0, vocab, 32).astype(np.int32)
+    bufs = [backend.HipBuffer.from_host(dev, a) for a in (lg, valid, recent)]
+    for k in (1, 2, 40, 64):
+        for scoring, temp in ((0, 0.9), (1, 20.0)):
+            check_select(backend, dev, orc, *bufs, lg, valid, recent, scoring, 9, temp, 77 + k, k,
+                         f"vocab={vocab} {shape} k={k} scoring={scoring}")
+
+
 def partition_bounds(vocab: int, parts: int, p: int):
     return vocab * p // parts, vocab * (p + 1) // parts
 
