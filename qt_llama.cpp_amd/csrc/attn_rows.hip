@@ -63,8 +63,6 @@ __device__ __forceinline__ void scalar_wait()
 // chain rows M at a time, lane p the chain of position T0 + p.  Chain row c of
 // a kv head is row c / G, head c % G of the group.  Row blocks are taken in
 // reverse order: the latest rows, with the most tiles, are dispatched first.
-constexpr int kRowsP = 64;   // positions per tile
-constexpr int kRowsW = 4;    // waves per workgroup
 __host__ __device__ constexpr int rows_k_stride(int head_dim) { return head_dim * 2 + 16; }
 
 template <int M>
@@ -193,7 +191,6 @@ __global__ __launch_bounds__(64 * kRowsW) void attn_rows_scores_kernel(
 // kRowsQC chain rows a pass, `reps` passes, four a wave.  One row a workgroup
 // spent ten times its dots on that re-laying: 300 rows x 8 heads of 256 dims
 // over a window of 512 took 143 us.
-constexpr int kRowsQM = 4, kRowsQC = kRowsW * kRowsQM;  // chain rows a wave, a pass
 __host__ __device__ constexpr int rows_q_kstride(int kf, int nb) { return nb * (kf == 2 ? 4 : 8) + 1; }  // dwords
 inline size_t rows_q_lds(int kf, int nb)
 {
@@ -635,20 +632,13 @@ __global__ __launch_bounds__(256) void attn_rows_pv_kernel(const float *__restri
 
 }  // namespace
 
-int launch_attn_rows_scores(mrml_hip_ctx *ctx, const float *q, int q_stride, const void *k_cache, int n_past0, int rows,
-                            int n_heads, int n_kv_heads, int head_dim, int k_fmt, float scale, int capacity, int wlimit,
-                            float *scores)
+int launch_attn_rows_scores(mrml_hip_ctx *ctx, const AttnRowsPlan &plan, const float *q, int q_stride,
+                            const void *k_cache, int n_past0, int rows, int n_heads, int n_kv_heads, int head_dim,
+                            int k_fmt, float scale, int capacity, int wlimit, float *scores)
 {
-    const int G = n_heads / n_kv_heads, nchains = rows * G;
-    // positions tiled absolutely from row 0's window start to the last row's position
-    const int count0 = n_past0 + 1, t_lo = count0 > wlimit ? count0 - wlimit : 0, t_hi = n_past0 + rows - 1;
-    const int tiles = (t_hi - t_lo) / kRowsP + 1;
-    const int64_t chain_tiles = (int64_t)tiles * n_kv_heads * nchains;
+    const int nchains = rows * (n_heads / n_kv_heads), t_lo = plan.t_lo, reps = plan.score_reps;
+    const dim3 grid((unsigned)plan.tiles, (unsigned)n_kv_heads, (unsigned)plan.score_blocks(nchains));
     if (k_fmt != 0) {
-        // passes over a staged tile: as many as leave four workgroups a CU
-        const int reps = (int)std::min<int64_t>(8, std::max<int64_t>(1, chain_tiles / (kRowsQC * 1024)));
-        const int per = kRowsQC * reps;
-        const dim3 grid((unsigned)tiles, (unsigned)n_kv_heads, (unsigned)((nchains + per - 1) / per));
 #define ROWS_SCQ(KF)                                                                                               \
     hipLaunchKernelGGL(attn_rows_scores_q_kernel<KF>, grid, dim3(64 * kRowsW), rows_q_lds(KF, head_dim / 32),       \
                        ctx->stream, q, q_stride, (const uint8_t *)k_cache, n_past0, nchains, n_heads, n_kv_heads,   \
@@ -658,48 +648,28 @@ int launch_attn_rows_scores(mrml_hip_ctx *ctx, const float *q, int q_stride, con
 #undef ROWS_SCQ
         return check_launch(ctx, "attn_rows_scores_q_kernel");
     }
-    // Chain rows a wave: four while that leaves two waves a SIMD, else two or
-    // one (77 rows of 8 heads at 377 positions: 9.6 us with one, 11 with four).
-    // Two sets of them a workgroup once the launch is many rounds of the chip
-    // (512 rows behind 2048 positions: 10,240 workgroups, 7 us less; 512 rows
-    // from the start: 2048, 2 us more).
-    const int M = chain_tiles >= 4 * 2048 ? 4 : (chain_tiles >= 2 * 2048 ? 2 : 1);
-    const int reps = chain_tiles / (kRowsW * M) >= 8192 ? 2 : 1;
-    const int per = kRowsW * M * reps;
-    const dim3 grid((unsigned)tiles, (unsigned)n_kv_heads, (unsigned)((nchains + per - 1) / per));
     const size_t lds = (size_t)kRowsP * rows_k_stride(head_dim);
 #define ROWS_SC(M)                                                                                               \
     hipLaunchKernelGGL(attn_rows_scores_kernel<M>, grid, dim3(64 * kRowsW), lds, ctx->stream, q, q_stride,          \
                        (const uint16_t *)k_cache, n_past0, nchains, n_heads, n_kv_heads, head_dim, scale, capacity, \
                        wlimit, t_lo, reps, scores)
-    if (M == 4) ROWS_SC(4);
-    else if (M == 2) ROWS_SC(2);
+    if (plan.score_m == 4) ROWS_SC(4);
+    else if (plan.score_m == 2) ROWS_SC(2);
     else ROWS_SC(1);
 #undef ROWS_SC
     return check_launch(ctx, "attn_rows_scores_kernel");
 }
 
-// The weighted sum reads the cache through one buffer descriptor (32-bit offsets).
-bool attn_rows_v_ok(int n_kv_heads, int head_dim, int v_fmt, int capacity)
-{
-    const uint64_t block = v_fmt == 0 ? 64 : (v_fmt == 1 ? 34 : 18);
-    return (uint64_t)capacity * n_kv_heads * (head_dim / 32) * block < (1ull << 32) - (1 << 20);
-}
-
 // Softmax in place over the scores, then the weighted sum of values.
-int launch_attn_rows_softmax_v(mrml_hip_ctx *ctx, float *scores, const void *v_cache, float *out, int n_past0, int rows,
-                               int n_heads, int n_kv_heads, int head_dim, int v_fmt, int capacity, int wlimit)
+int launch_attn_rows_softmax_v(mrml_hip_ctx *ctx, const AttnRowsPlan &plan, float *scores, const void *v_cache,
+                               float *out, int n_past0, int rows, int n_heads, int n_kv_heads, int head_dim, int v_fmt,
+                               int capacity, int wlimit)
 {
-    const int fe = (int)host_expf_fused(), span = std::min(wlimit, n_past0 + rows);
+    const int fe = (int)host_expf_fused(), nt = plan.softmax_threads;
     const dim3 sgrid((unsigned)n_heads, (unsigned)rows);
 #define ROWS_SM(NT)                                                                                              \
     hipLaunchKernelGGL(attn_rows_softmax_kernel<NT>, sgrid, dim3(NT), 0, ctx->stream, scores, n_past0, n_heads,   \
                        capacity, wlimit, fe)
-    // Rows enough to fill the chip: small workgroups, more of them a CU, and
-    // chunks past 1024 positions (512 rows x 8 heads of 2300 positions: 54 us,
-    // 65 with 512 threads, 76 with 1024).  Few rows: the latency of one chunk
-    // counts (4 rows of 3000 positions: 6 us with 1024 threads, 13 with 256).
-    const int nt = span <= 1024 || (int64_t)rows * n_heads >= 1024 ? 256 : (span <= 2048 ? 512 : 1024);
     if (nt == 256) ROWS_SM(256);
     else if (nt == 512) ROWS_SM(512);
     else ROWS_SM(1024);
@@ -707,9 +677,6 @@ int launch_attn_rows_softmax_v(mrml_hip_ctx *ctx, float *scores, const void *v_c
     if (int rc = check_launch(ctx, "attn_rows_softmax_kernel")) return rc;
 
     const int nchains = rows * (n_heads / n_kv_heads);
-    auto waves = [&](int m, int d) {
-        return (int64_t)n_kv_heads * ((nchains + m - 1) / m) * ((head_dim + 64 * d - 1) / (64 * d));
-    };
     const uint8_t *v = reinterpret_cast<const uint8_t *>(v_cache);
 #define ROWS_PV(VF, M, D)                                                                                          \
     do {                                                                                                           \
@@ -720,23 +687,11 @@ int launch_attn_rows_softmax_v(mrml_hip_ctx *ctx, float *scores, const void *v_c
     } while (0)
 #define ROWS_PV_MD(VF)                                                                                             \
     do {                                                                                                           \
-        if (form == 0) ROWS_PV(VF, 4, 2);                                                                          \
-        else if (form == 1) ROWS_PV(VF, 4, 1);                                                                     \
-        else if (form == 2) ROWS_PV(VF, 2, 1);                                                                     \
+        if (plan.pv_m == 4 && plan.pv_d == 2) ROWS_PV(VF, 4, 2);                                                   \
+        else if (plan.pv_m == 4) ROWS_PV(VF, 4, 1);                                                                \
+        else if (plan.pv_m == 2) ROWS_PV(VF, 2, 1);                                                                \
         else ROWS_PV(VF, 1, 1);                                                                                    \
     } while (0)
-    // The widest form that leaves waves enough: the four-row forms issue the
-    // fewest conversions and loads a product, the narrow ones keep more SIMDs
-    // busy.  us at (4,2) / (4,1) / (2,1) / (1,1), whole attention, waves of the
-    // first: 512 rows behind 2048 (2048) 347 / 364 / 490 / 741; 333 rows from
-    // 0 (1332) 46.3 / 43.5 / 47.3 / 61; 77 rows behind 300 (308) 37.6 / 32.6 /
-    // 31.3 / 36.2; 200 rows of 4 x 64 dims, window 512 (200) 46 / 40 / 33 / 29.
-    // Quantised rows cost more a load: 300 rows of 8 x 128 Q8_0 (600) 196 /
-    // 233 / 223 / 292.
-    const int form = waves(4, 2) >= (v_fmt == 0 ? 2048 : 600) ? 0
-                     : waves(4, 1) >= 800                      ? 1
-                     : waves(2, 1) >= 800                      ? 2
-                                                               : 3;
     if (v_fmt == 0) ROWS_PV_MD(0);
     else if (v_fmt == 1) ROWS_PV_MD(1);
     else ROWS_PV_MD(2);

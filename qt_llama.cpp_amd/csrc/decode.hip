@@ -788,7 +788,6 @@ __global__ __launch_bounds__(kScoreT) void attn_scores2_kernel(const float *__re
 // tile, products double-buffered).
 // Writes out (nullable) and the Q8_0 pack of the n_heads*head_dim output
 // (nullable).  Dynamic LDS: a float a position of the widest window (sv_lds).
-constexpr int kSVD = 32;  // dims per workgroup
 constexpr int kSVW = 8;   // waves: wave 0 adds; waves 1-3 and 5-7 produce; wave 4, which shares wave 0's SIMD, idles
 constexpr int kSVT = 96;  // positions per tile: 48 position pairs x 8 dim quads = one per producer thread
 constexpr int kSVS = kSVT + 12;  // product row stride (floats), 27 16-byte segments: measured on gfx950, 16-byte
@@ -897,18 +896,9 @@ __device__ __forceinline__ void sv_products(const u32x2 (&r)[kSVR], const float 
 // equal the one sequential loop), and the producers form their weights from
 // the global scores.  Dynamic LDS: kSVChunk floats, kSVChunk flag bytes and
 // the block sum's Shared.
-//
-// The line lies on the widest window of the launch, not on the cache's
-// capacity, and where the weights take as much LDS as LONG's chunk and flags:
-// up to there the LDS form costs no resident workgroup.  Attention in caches
-// of 8192 positions, LONG / LDS form: 5310 positions, 4 heads of 64 dims over
-// Q4_0 rows 65.6 / 41.9 us; 2774, 8 heads of 128 over f16 36.8 / 25.4; a window
-// of 1024, 16 heads of 128 over Q8_0/Q4_0 23.2 / 19.5.
-constexpr int kSVShort = 10240;  // positions: 40 KiB of weights
 constexpr int kSVChunk = 8192;     // LONG: terms per exact block sum (16 per thread)
 static_assert(kSVChunk <= mrml_xsum::kMaxPerThread * 64 * kSVW, "one block sum per chunk");
 
-__host__ __device__ constexpr bool sv_long(int span) { return span > kSVShort; }
 inline size_t sv_lds(int span)  // (weights are read in pairs)
 {
     return sv_long(span) ? (size_t)kSVChunk * 5 + sizeof(mrml_xsum::Shared)
@@ -1681,25 +1671,16 @@ int launch_attn_rows(mrml_hip_ctx *ctx, const float *q, int q_stride, const void
                      float scale, int capacity, void *scratch, int sliding_window)
 {
     float *scores = reinterpret_cast<float *>(scratch);
-    const int wlimit = attn_window_limit(capacity, sliding_window), span = std::min(wlimit, n_past0 + rows);
-    if (int rc = launch_attn_rows_scores(ctx, q, q_stride, k_cache, n_past0, rows, n_heads, n_kv_heads, head_dim, k_fmt,
-                                         scale, capacity, wlimit, scores))
+    const int wlimit = attn_window_limit(capacity, sliding_window);
+    const AttnRowsPlan plan = attn_rows_plan(n_past0, rows, n_heads, n_kv_heads, head_dim, k_fmt, v_fmt, capacity, wlimit);
+    if (int rc = launch_attn_rows_scores(ctx, plan, q, q_stride, k_cache, n_past0, rows, n_heads, n_kv_heads, head_dim,
+                                         k_fmt, scale, capacity, wlimit, scores))
         return rc;
-    // The decode form's workgroup adds 32 dims of one row at 4.7 ns a
-    // position, the rows form's waves need company for that: while the decode
-    // form's workgroups are all resident at once (three or four a CU) and its
-    // repeated softmax is not what they spend their time on, it is the faster.
-    // Measured (us, decode form / rows form, 8 heads): 8 rows x 256 dims (512
-    // workgroups) at 300 positions 20 / 22, at 3000 75 / 83; 12 rows (768) at
-    // 300 25 / 22; 60 rows x 64 dims (960) at 1000 54 / 66; 20 rows x 256
-    // (1280) at 512 47 / 44; 32 rows (2048) at 100 44 / 19.
-    const int64_t wgs = (int64_t)rows * n_heads * (head_dim / kSVD);
-    if (wgs <= 512 || (wgs <= 1024 && span > 512) ||
-        !attn_rows_v_ok(n_kv_heads, head_dim, v_fmt, capacity))
+    if (!plan.rows_form)
         return launch_softmax_v(ctx, scores, v_cache, out, nullptr, nullptr, n_past0, n_heads, n_kv_heads, capacity,
                                 wlimit, rows, head_dim, v_fmt);
-    return launch_attn_rows_softmax_v(ctx, scores, v_cache, out, n_past0, rows, n_heads, n_kv_heads, head_dim, v_fmt,
-                                      capacity, wlimit);
+    return launch_attn_rows_softmax_v(ctx, plan, scores, v_cache, out, n_past0, rows, n_heads, n_kv_heads, head_dim,
+                                      v_fmt, capacity, wlimit);
 }
 
 int launch_rope_kv_any(mrml_hip_ctx *ctx, float *qkv, void *k_cache, void *v_cache, int pos, int n_heads,

@@ -60,14 +60,12 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kGemmWaves = 4;             // 32-token groups per workgroup, sharing one 32-row tile
 constexpr int kPF = 4;                    // B prefetch distance, blocks
 constexpr int kKC = 8;                    // blocks per A chunk
 constexpr int kNBuf = 3;                  // A chunk buffers in LDS
 constexpr int kBufferFlags = 0x00020000;  // buffer resource word 3 (raw 32-bit data) on gfx9
 constexpr float kMagic = 12582912.0f;      // 1.5 * 2^23
 constexpr int kMagicBits = 0x4B400000;     // its f32 bit pattern
-constexpr int kSIMDs = 1024;               // MI355X: 256 CUs x 4 SIMDs
 
 // quant.rs:193-228 per block (q8_0_block8x4), written as a GEMM pack.  One
 // workgroup per (group, block): thread 8t+l handles token 32g+t, values
@@ -429,7 +427,6 @@ __global__ __launch_bounds__(64 * kGemmWaves) void gemm_q4_0_mfma_kernel(const G
 //     blocks), and the same transpose gives quarter q dword q of both halves;
 //   token scales: lane 16q + 4b + e loads token 4q + e of block b, which the
 //     scale products read as a row broadcast (a DPP operand, no instruction).
-constexpr int kFewRows = 16, kFewTokens = 16;
 constexpr int kFewAdders = 4;  // waves; kFewRows * kFewTokens lanes
 
 // Quarter q of a: dword q of block j for j = 0..3, from quarter p holding dwords 0..3 of block p.
@@ -709,38 +706,15 @@ int launch_gemm_pack_from_act(mrml_hip_ctx *ctx, const void *pack, void *gpack, 
     return check_launch(ctx, "gemm_pack_from_act_kernel");
 }
 
-static int few_workgroups(int32_t rows, int32_t batch)
-{
-    return (rows + kFewRows - 1) / kFewRows * ((batch + kFewTokens - 1) / kFewTokens);
-}
-
-// Whether a product runs as gemm_q4_0_few_kernel.  A workgroup costs about
-// 8.5e-5 us a block there once the chip is full; the tile kernel takes 0.2 us
-// a block for anything up to one wave a SIMD (a lone wave's step), so the
-// line is at 0.2 / 8.5e-5 workgroups.  Measured on both sides of it:
-// 9216 x 2304 at 64 tokens (2304 workgroups) 17.6 against 19.7 us, at 80
-// (2880) 21.4 against 20.0; 4096 x 2304 at 128 (2048) 15.5 against 18.1;
-// 2304 x 9216 at 128 (1152) 28.4 against 58.7.
-bool gemm_few(int32_t rows, int32_t batch)
-{
-    return (int64_t)(rows + kFewRows - 1) / kFewRows * ((batch + kFewTokens - 1) / kFewTokens) <= 2304;
-}
-
-// Producers: 8 while the workgroups leave CUs their LDS (two of them a CU),
-// else 4 (up to four a CU).  2304 x 9216 at 16 tokens (144 workgroups) 9.6
-// with 8, 12.6 us with 4; at 48 (432) 13.8 and 15.0; 4096 x 2304 at 24 (512)
-// 7.1 and 6.4.  GLU holds two products' terms, so it takes 4: 9216 x 2304 at
-// 12 tokens 16.2 us, 21.0 with 8 (two tile products and the elementwise pass:
-// 42.5).
 static int launch_gemm_few(mrml_hip_ctx *ctx, bool glu, const GemmMats &mats, const void *gpack, float *y,
                            int32_t rows, int nb, int32_t batch, int32_t ldy)
 {
-    const int ng = gemm_groups(batch), wgs = few_workgroups(rows, batch);
-    const dim3 grid((unsigned)wgs);
+    const int ng = gemm_groups(batch);
+    const dim3 grid((unsigned)few_workgroups(rows, batch));
     if (glu)
         hipLaunchKernelGGL((gemm_q4_0_few_kernel<true, 4>), grid, dim3(64 * (kFewAdders + 4)), 0, ctx->stream, mats,
                            (const uint8_t *)gpack, y, rows, nb, batch, ng, ldy);
-    else if (wgs < 448)
+    else if (gemm_few_producers(false, rows, batch) == 8)
         hipLaunchKernelGGL((gemm_q4_0_few_kernel<false, 8>), grid, dim3(64 * (kFewAdders + 8)), 0, ctx->stream, mats,
                            (const uint8_t *)gpack, y, rows, nb, batch, ng, ldy);
     else
@@ -759,16 +733,8 @@ static int launch_gemm_mats(mrml_hip_ctx *ctx, const GemmMats &mats, const void 
                     ldy, rows);
     if (!relaxed && gemm_few(rows, batch)) return launch_gemm_few(ctx, false, mats, gpack, y, rows, nb, batch, ldy);
     const int vec = (ldy % 4 == 0 && ((uintptr_t)y & 15) == 0) ? 1 : 0;  // float4 stores reach every output row
-    // FULL waves, one per (row tile, token group).  When they number just
-    // over one per SIMD (down at M = 512: 1152 for 1024), the SIMDs holding
-    // two of them set the launch's time; then only as many row tiles as
-    // give every SIMD one FULL wave stay FULL and the rest run as HALF waves
-    // (two per token group), which add a little over half a wave's work to
-    // some SIMDs instead of a whole one.
     const int rt = (rows + 31) / 32, gq = (ng + kGemmWaves - 1) / kGemmWaves;
-    const int full_waves = rt * gq * kGemmWaves;
-    int rt_full = rt;
-    if (full_waves > kSIMDs && 2 * full_waves <= 3 * kSIMDs) rt_full = kSIMDs / (gq * kGemmWaves);
+    const int rt_full = gemm_full_tiles(rows, batch);
     const int hq = (2 * ng + kGemmWaves - 1) / kGemmWaves;  // workgroups of HALF waves per row tile
     const dim3 grid((unsigned)(rt_full * gq + (rt - rt_full) * hq));
     if (relaxed)

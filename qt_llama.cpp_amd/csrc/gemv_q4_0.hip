@@ -1511,7 +1511,6 @@ static int iters_round(int iters)
 constexpr int kFoldWaves = 4;   // fold16 compute waves per workgroup
 constexpr int kRelayS = 6;      // relay waves per 4 rows for 288-block rows (gate/up pairs)
 constexpr int kLongS = 3;       // compute waves per 4 rows of the long-row kernel
-constexpr int kCUs = 256;       // MI355X compute units: workgroup counts that divide among them evenly
 
 inline bool fold16_shape(int nb) { return nb == 64 || nb == 72; }
 inline bool relay_shape(int nb) { return nb == 288; }

@@ -7,6 +7,7 @@
 #include <string>
 
 #include "../../include/mrml_hip.h"
+#include "plans.h"
 
 struct mrml_hip_ctx {
     int32_t device = 0;
@@ -112,9 +113,6 @@ int launch_gemm_q4_0(mrml_hip_ctx *ctx, const void *w, const void *gpack, float 
                      int32_t batch, int32_t ldy = 0, bool relaxed = false);
 int launch_gemm_q4_0_stacked(mrml_hip_ctx *ctx, const void *const *w, const int32_t *rows, int n, const void *gpack,
                              float *y, int32_t cols, int32_t batch, int32_t ldy, bool relaxed = false);
-// Whether an exact product of this size takes the few-token kernel (a relaxed one never does: the tile
-// kernel's one-FMA fold is slower there than the few-token kernel's exact one).
-bool gemm_few(int32_t rows, int32_t batch);
 // act = gelu_tanh(Wg x) * (Wu x) of every token ([batch][rows], unpadded rows); gu: 2*batch*rows floats of scratch
 int launch_gemm_q4_0_geglu(mrml_hip_ctx *ctx, const void *wg, const void *wu, const void *gpack, float *act, float *gu,
                            int32_t rows, int32_t cols, int32_t batch);
@@ -217,14 +215,13 @@ bool attn_rope_ok(int n_heads, int n_kv_heads);
 int launch_attn_rows(mrml_hip_ctx *ctx, const float *q, int q_stride, const void *k_cache, const void *v_cache,
                      float *out, int n_past0, int rows, int n_heads, int n_kv_heads, int head_dim, int k_fmt, int v_fmt,
                      float scale, int capacity, void *scratch, int sliding_window);
-// Its parts in attn_rows.hip: scores; softmax and weighted sum
-// (caches that attn_rows_v_ok says a buffer descriptor reaches).
-int launch_attn_rows_scores(mrml_hip_ctx *ctx, const float *q, int q_stride, const void *k_cache, int n_past0, int rows,
-                            int n_heads, int n_kv_heads, int head_dim, int k_fmt, float scale, int capacity, int wlimit,
-                            float *scores);
-bool attn_rows_v_ok(int n_kv_heads, int head_dim, int v_fmt, int capacity);
-int launch_attn_rows_softmax_v(mrml_hip_ctx *ctx, float *scores, const void *v_cache, float *out, int n_past0, int rows,
-                               int n_heads, int n_kv_heads, int head_dim, int v_fmt, int capacity, int wlimit);
+// Its parts in attn_rows.hip, in the forms of attn_rows_plan (plans.h): scores; softmax and weighted sum.
+int launch_attn_rows_scores(mrml_hip_ctx *ctx, const AttnRowsPlan &plan, const float *q, int q_stride,
+                            const void *k_cache, int n_past0, int rows, int n_heads, int n_kv_heads, int head_dim,
+                            int k_fmt, float scale, int capacity, int wlimit, float *scores);
+int launch_attn_rows_softmax_v(mrml_hip_ctx *ctx, const AttnRowsPlan &plan, float *scores, const void *v_cache,
+                               float *out, int n_past0, int rows, int n_heads, int n_kv_heads, int head_dim, int v_fmt,
+                               int capacity, int wlimit);
 // Attention over caches of any head size (a multiple of 32 up to 512),
 // groups of up to 16 and the KV formats 0 (f16), 1 (Q8_0), 2 (Q4_0):
 // one query at position n_past (or *d_pos), the arithmetic of the CPU loop

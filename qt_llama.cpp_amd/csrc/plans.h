@@ -1,0 +1,164 @@
+// plans.h -- which kernel form a batched attention, a decode softmax or a
+// batched product takes: the dispatch rules as host functions of sizes, types
+// and positions (no HIP in here, so that a CPU test can evaluate them).
+#pragma once
+
+#include <stddef.h>
+#include <stdint.h>
+
+#include <algorithm>
+
+namespace mrml {
+
+constexpr int kCUs = 256, kSIMDs = 4 * kCUs;  // MI355X
+
+// ---- decode softmax ------------------------------------------------------------
+// The line lies on the widest window of the launch, not on the cache's
+// capacity, and where the weights take as much LDS as LONG's chunk and flags:
+// up to there the LDS form costs no resident workgroup.  Attention in caches
+// of 8192 positions, LONG / LDS form: 5310 positions, 4 heads of 64 dims over
+// Q4_0 rows 65.6 / 41.9 us; 2774, 8 heads of 128 over f16 36.8 / 25.4; a window
+// of 1024, 16 heads of 128 over Q8_0/Q4_0 23.2 / 19.5.
+constexpr int kSVShort = 10240;  // positions: 40 KiB of weights
+#if defined(__HIPCC__)
+__host__ __device__
+#endif
+constexpr bool sv_long(int span) { return span > kSVShort; }
+
+constexpr int kSVD = 32;  // dims of a decode-form workgroup
+
+// ---- attention of many query rows ------------------------------------------------
+// `rows` rows at positions n_past0.., each seeing the last min(position + 1,
+// wlimit) positions.
+constexpr int kRowsP = 64;    // positions per score tile
+constexpr int kRowsW = 4;     // waves per score workgroup
+constexpr int kRowsQM = 4, kRowsQC = kRowsW * kRowsQM;  // quantised K: chain rows a wave, a pass
+
+struct AttnRowsPlan {
+    int span;        // the widest window
+    int t_lo;        // the first row's window start
+    int tiles;       // score tiles from there to the last row's position
+    int score_m;     // chain rows (row x query head) a wave
+    int score_reps;  // passes over a staged tile
+    bool rows_form;  // softmax and weighted sum as attn_rows.hip has them, else the decode form
+    int softmax_threads;
+    int pv_m, pv_d;  // weighted sum: chain rows a wave, dims a lane
+    int score_blocks(int nchains) const
+    {
+        const int per = kRowsW * score_m * score_reps;
+        return (nchains + per - 1) / per;
+    }
+};
+
+// The weighted sum of the rows form reads the cache through one buffer descriptor (32-bit offsets).
+inline bool attn_rows_v_ok(int n_kv_heads, int head_dim, int v_fmt, int capacity)
+{
+    const uint64_t block = v_fmt == 0 ? 64 : (v_fmt == 1 ? 34 : 18);
+    return (uint64_t)capacity * n_kv_heads * (head_dim / 32) * block < (1ull << 32) - (1 << 20);
+}
+
+inline AttnRowsPlan attn_rows_plan(int n_past0, int rows, int n_heads, int n_kv_heads, int head_dim, int k_fmt,
+                                   int v_fmt, int capacity, int wlimit)
+{
+    AttnRowsPlan p{};
+    const int nchains = rows * (n_heads / n_kv_heads), count0 = n_past0 + 1;
+    p.span = std::min(wlimit, n_past0 + rows);
+    // positions tiled absolutely from row 0's window start to the last row's position
+    p.t_lo = count0 > wlimit ? count0 - wlimit : 0;
+    p.tiles = (n_past0 + rows - 1 - p.t_lo) / kRowsP + 1;
+    const int64_t chain_tiles = (int64_t)p.tiles * n_kv_heads * nchains;
+    if (k_fmt != 0) {
+        // passes over a staged tile: as many as leave four workgroups a CU
+        p.score_m = kRowsQM;
+        p.score_reps = (int)std::min<int64_t>(8, std::max<int64_t>(1, chain_tiles / (kRowsQC * 4 * kCUs)));
+    } else {
+        // Chain rows a wave: four while that leaves two waves a SIMD, else two or
+        // one (77 rows of 8 heads at 377 positions: 9.6 us with one, 11 with four).
+        // Two sets of them a workgroup once the launch is many rounds of the chip
+        // (512 rows behind 2048 positions: 10,240 workgroups, 7 us less; 512 rows
+        // from the start: 2048, 2 us more).
+        p.score_m = chain_tiles >= 4 * 2 * kSIMDs ? 4 : (chain_tiles >= 2 * 2 * kSIMDs ? 2 : 1);
+        p.score_reps = chain_tiles / (kRowsW * p.score_m) >= 8192 ? 2 : 1;
+    }
+
+    // The decode form's workgroup adds 32 dims of one row at 4.7 ns a
+    // position, the rows form's waves need company for that: while the decode
+    // form's workgroups are all resident at once (three or four a CU) and its
+    // repeated softmax is not what they spend their time on, it is the faster.
+    // Measured (us, decode form / rows form, 8 heads): 8 rows x 256 dims (512
+    // workgroups) at 300 positions 20 / 22, at 3000 75 / 83; 12 rows (768) at
+    // 300 25 / 22; 60 rows x 64 dims (960) at 1000 54 / 66; 20 rows x 256
+    // (1280) at 512 47 / 44; 32 rows (2048) at 100 44 / 19.
+    const int64_t wgs = (int64_t)rows * n_heads * (head_dim / kSVD);
+    p.rows_form = !(wgs <= 512 || (wgs <= 1024 && p.span > 512)) &&
+                  attn_rows_v_ok(n_kv_heads, head_dim, v_fmt, capacity);
+
+    // Rows enough to fill the chip: small workgroups, more of them a CU, and
+    // chunks past 1024 positions (512 rows x 8 heads of 2300 positions: 54 us,
+    // 65 with 512 threads, 76 with 1024).  Few rows: the latency of one chunk
+    // counts (4 rows of 3000 positions: 6 us with 1024 threads, 13 with 256).
+    p.softmax_threads = p.span <= 1024 || (int64_t)rows * n_heads >= 1024 ? 256 : (p.span <= 2048 ? 512 : 1024);
+
+    // The widest form that leaves waves enough: the four-row forms issue the
+    // fewest conversions and loads a product, the narrow ones keep more SIMDs
+    // busy.  us at (4,2) / (4,1) / (2,1) / (1,1), whole attention, waves of the
+    // first: 512 rows behind 2048 (2048) 347 / 364 / 490 / 741; 333 rows from
+    // 0 (1332) 46.3 / 43.5 / 47.3 / 61; 77 rows behind 300 (308) 37.6 / 32.6 /
+    // 31.3 / 36.2; 200 rows of 4 x 64 dims, window 512 (200) 46 / 40 / 33 / 29.
+    // Quantised rows cost more a load: 300 rows of 8 x 128 Q8_0 (600) 196 /
+    // 233 / 223 / 292.
+    auto waves = [&](int m, int d) {
+        return (int64_t)n_kv_heads * ((nchains + m - 1) / m) * ((head_dim + 64 * d - 1) / (64 * d));
+    };
+    p.pv_m = 1, p.pv_d = 1;
+    if (waves(4, 2) >= (v_fmt == 0 ? 2048 : 600)) p.pv_m = 4, p.pv_d = 2;
+    else if (waves(4, 1) >= 800) p.pv_m = 4;
+    else if (waves(2, 1) >= 800) p.pv_m = 2;
+    return p;
+}
+
+// ---- batched Q4_0 products ---------------------------------------------------------
+constexpr int kGemmWaves = 4;  // 32-token groups per workgroup of the tile kernel, sharing one 32-row tile
+constexpr int kFewRows = 16, kFewTokens = 16;  // of a few-token workgroup
+
+inline int64_t few_workgroups(int32_t rows, int32_t batch)
+{
+    return (int64_t)((rows + kFewRows - 1) / kFewRows) * ((batch + kFewTokens - 1) / kFewTokens);
+}
+
+// Whether an exact product runs as gemm_q4_0_few_kernel (a relaxed one never
+// does: the tile kernel's one-FMA fold is slower there than the few-token
+// kernel's exact one).  A workgroup costs about 8.5e-5 us a block there once
+// the chip is full; the tile kernel takes 0.2 us a block for anything up to
+// one wave a SIMD (a lone wave's step), so the line is at 0.2 / 8.5e-5
+// workgroups.  Measured on both sides of it:
+// 9216 x 2304 at 64 tokens (2304 workgroups) 17.6 against 19.7 us, at 80
+// (2880) 21.4 against 20.0; 4096 x 2304 at 128 (2048) 15.5 against 18.1;
+// 2304 x 9216 at 128 (1152) 28.4 against 58.7.
+inline bool gemm_few(int32_t rows, int32_t batch) { return few_workgroups(rows, batch) <= 2304; }
+
+// Producers of a few-token workgroup: 8 while the workgroups leave CUs their
+// LDS (two of them a CU), else 4 (up to four a CU).  2304 x 9216 at 16 tokens
+// (144 workgroups) 9.6 with 8, 12.6 us with 4; at 48 (432) 13.8 and 15.0; 4096
+// x 2304 at 24 (512) 7.1 and 6.4.  GLU holds two products' terms, so it takes
+// 4: 9216 x 2304 at 12 tokens 16.2 us, 21.0 with 8 (two tile products and the
+// elementwise pass: 42.5).
+inline int gemm_few_producers(bool glu, int32_t rows, int32_t batch)
+{
+    return !glu && few_workgroups(rows, batch) < 448 ? 8 : 4;
+}
+
+// Row tiles that the tile kernel runs as FULL waves, one per (row tile, token
+// group).  When those number just over one per SIMD (2304 rows at 512 tokens:
+// 1152 for 1024), the SIMDs holding two of them set the launch's time; then
+// only as many row tiles as give every SIMD one FULL wave stay FULL and the
+// rest run as HALF waves (two per token group), which add a little over half a
+// wave's work to some SIMDs instead of a whole one.
+inline int gemm_full_tiles(int32_t rows, int32_t batch)
+{
+    const int ng = (batch + 31) / 32, rt = (rows + 31) / 32, gq = (ng + kGemmWaves - 1) / kGemmWaves;
+    const int64_t full_waves = (int64_t)rt * gq * kGemmWaves;
+    return full_waves > kSIMDs && 2 * full_waves <= 3 * kSIMDs ? kSIMDs / (gq * kGemmWaves) : rt;
+}
+
+}  // namespace mrml

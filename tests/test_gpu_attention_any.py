@@ -216,7 +216,7 @@ def test_attention_prefill_any(backend, dev, orc, nh, nkv, hd, kf, vf):
 # one position), the ring's end inside the window, capacities below a tile,
 # softmax rows of one chunk and of several (1024 rows x heads and more past
 # 1024 positions), and the decode form's side of the line.
-@pytest.mark.parametrize("nh,nkv,hd,kf,vf,cap,sw,start,batch", [
+MANY_ROWS = [
     (8, 4, 256, 0, 0, 1024, None, 300, 300),   # 4x1, tail batches of every length
     (8, 4, 256, 0, 0, 2048, None, 0, 513),     # 4x2, from position 0
     (8, 4, 256, 0, 0, 256, None, 500, 77),     # 2x1, the ring wrapped
@@ -231,7 +231,23 @@ def test_attention_prefill_any(backend, dev, orc, nh, nkv, hd, kf, vf):
     (6, 2, 96, 2, 2, 300, 130, 280, 130),      # 2x1
     (8, 4, 256, 0, 0, 512, None, 100, 8),      # decode form (512 workgroups)
     (8, 4, 256, 0, 0, 512, None, 100, 9),
-])
+    (8, 4, 256, 0, 0, 4096, None, 2048, 512),  # two passes over a staged score tile
+    (8, 4, 256, 1, 1, 1024, None, 100, 460),   # the same over quantised K; Q8_0 at 4x2
+    (8, 4, 256, 2, 2, 1024, None, 100, 460),
+    (8, 4, 256, 2, 1, 512, None, 200, 120),    # Q8_0 at 4x1
+    (8, 4, 256, 1, 2, 512, None, 200, 110),    # Q4_0 at 4x1
+    (8, 2, 128, 1, 2, 512, 100, 200, 140),     # Q4_0 at 2x1
+    (8, 4, 256, 0, 0, 8192, None, 5000, 20),   # softmax in chunks of 1024 threads
+    (8, 4, 256, 1, 1, 512, None, 300, 6),      # decode form over quantised rows
+    (8, 2, 128, 2, 2, 512, 130, 300, 12),
+    # the long softmax with several rows, at every value format; the second and third across whole chunks
+    (4, 2, 64, 0, 0, 16384, None, 11000, 3),
+    (4, 2, 64, 1, 1, 16384, None, 16380, 4),
+    (2, 1, 96, 2, 2, 20000, 16382, 19000, 5),
+]
+
+
+@pytest.mark.parametrize("nh,nkv,hd,kf,vf,cap,sw,start,batch", MANY_ROWS)
 def test_attention_prefill_many_rows(backend, dev, orc, nh, nkv, hd, kf, vf, cap, sw, start, batch):
     kvd, qd = nkv * hd, nh * hd
     rng = np.random.default_rng(8250 + hd + cap + batch)
@@ -250,7 +266,7 @@ def test_attention_prefill_many_rows(backend, dev, orc, nh, nkv, hd, kf, vf, cap
     dev.attention_prefill(qb, kb, vb, out, start, batch, nh, nkv, hd, scale, sw, cap, kf, vf, q_stride=stride)
     dev.sync()
     got = out.numpy().reshape(batch, qd)
-    for i in sorted({*range(4), batch // 3, batch // 2, *range(batch - 5, batch)}):
+    for i in sorted({*range(min(4, batch)), batch // 3, batch // 2, *range(max(0, batch - 5), batch)}):
         ref = oracle_rows(orc, q[i * stride:i * stride + qd], kc, vc, start + i, sw, cap, nh, nkv, hd, scale, kf, vf)
         assert_bits(got[i], ref, f"row {i}")
 

@@ -247,53 +247,21 @@ def window_rows(n_past, sw, cap):
 # (cache_start, batch, sliding_window, capacity, n_heads, n_kv_heads, stacked q):
 # prefill_cuda's first chunk over the stacked projection, a later chunk, a
 # sliding window shorter than the chunk, a ring whose window covers the
-# whole capacity, a group of 8 query heads per kv head, the long softmax form
-# (capacity past 6144), a batch split over two launches (40 rows of 2 MiB of
-# scores against a 64 MiB bound), and windows past 2048 in the prefill
-# softmax form (groups of 2 and 4)
+# whole capacity, a group of 8 query heads per kv head, a window past 6000,
+# a batch split over two launches (40 rows of 2 MiB of scores against a
+# 64 MiB bound), and windows past 2048.  Which forms they and the many-row
+# cases of test_gpu_attention_any.py reach: test_plans.py.
 PREFILL_CASES = [(0, 16, None, 16, 8, 4, True), (128, 37, None, 512, 8, 4, True), (200, 40, 24, 256, 8, 4, True),
                  (300, 9, 64, 64, 8, 4, False), (700, 64, None, 2048, 8, 8, False), (20, 7, 5, 32, 16, 2, True),
                  (6000, 3, None, 8192, 8, 4, False), (100, 40, None, 65536, 8, 4, True),
                  (3000, 20, None, 4096, 8, 4, True), (3900, 9, None, 4096, 16, 4, False),
-                 # the rows form at groups of 4 and 3 (spans ~2000-4000)
+                 # groups of 4 and 3 (spans ~2000-4000)
                  (1990, 10, None, 4096, 16, 4, False), (3290, 10, None, 4096, 16, 4, True),
                  (2490, 12, None, 4096, 12, 4, False), (3990, 6, None, 4096, 12, 4, True),
-                 # windows up to 1024 (each thread's exps in registers) at groups
-                 # of 4 and 3, and both sides of that bound (spans 1024, 1025)
+                 # windows up to 1024 at groups of 4 and 3, and both sides of
+                 # that bound (spans 1024, 1025)
                  (500, 24, None, 4096, 16, 4, False), (900, 30, None, 1024, 12, 4, True),
                  (1000, 24, None, 4096, 8, 4, True), (1001, 24, None, 4096, 8, 4, False)]
-
-
-def prefill_span(cache_start, batch, sw, cap):
-    """The widest row window of a launch (launch_attn_rows_f16's span)."""
-    wlimit = sw if sw is not None and 0 < sw < cap else cap
-    return min(wlimit, cache_start + batch)
-
-
-def rows_form(nh, nkv, span):
-    """Whether attention_prefill runs attn_softmax_v_rows_kernel (the form
-    whose workgroup serves a kv head's whole group) rather than the
-    per-head attn_softmax_v_kernel: windows up to 4096, groups up to 4, and
-    the group's weights (a row of span floats per head, at a stride rounded
-    up to 4 floats) plus span flag bytes within 60 KiB of dynamic LDS
-    (launch_attn_rows_f16 in decode.hip)."""
-    g = nh // nkv
-    return span <= 4096 and g <= 4 and g * ((span + 3) & ~3) * 4 + ((span + 15) & ~15) <= 60 << 10
-
-
-def test_prefill_cases_cover_both_forms():
-    """The case list reaches the rows form at every group size it serves
-    (1, 2, 3, 4) and the per-head form too, so no group size is covered
-    only by a silent fallback."""
-    forms = {}
-    for start, batch, sw, cap, nh, nkv, _ in PREFILL_CASES:
-        forms.setdefault((nh // nkv, rows_form(nh, nkv, prefill_span(start, batch, sw, cap))), []).append(start)
-    for g in (1, 2, 3, 4):
-        assert (g, True) in forms, f"no attention_prefill case takes the rows form at group {g}"
-    assert any(not rows for _, rows in forms), "no case takes the per-head form"
-    # the two group-of-4 and group-of-3 cases above are rows-form cases
-    for start, batch, sw, cap, nh, nkv, _ in PREFILL_CASES[-4:]:
-        assert rows_form(nh, nkv, prefill_span(start, batch, sw, cap))
 
 
 @pytest.mark.parametrize("cache_start,batch,sw,cap,nh,nkv,stacked", PREFILL_CASES)
@@ -307,9 +275,8 @@ def test_attention_prefill_bit_exact(backend, dev, orc, cache_start, batch, sw, 
     vc = rng.standard_normal(cap * kvd).astype(np.float16).view(np.uint16)
     qb, kb, vb = (backend.HipBuffer.from_host(dev, a) for a in (q, kc, vc))
     out = backend.HipBuffer.alloc(dev, batch * qd)
-    form = "rows" if rows_form(nh, nkv, prefill_span(cache_start, batch, sw, cap)) else "per-head"
-    print(f"\n[attention_prefill] start {cache_start} batch {batch} window {sw} capacity {cap} heads {nh}/{nkv} "
-          f"({form} form)", flush=True)
+    print(f"\n[attention_prefill] start {cache_start} batch {batch} window {sw} capacity {cap} heads {nh}/{nkv}",
+          flush=True)
     dev.attention_prefill(qb, kb, vb, out, cache_start, batch, nh, nkv, hd, 1.0 / 16.0, sw, cap)
     dev.sync()
     got = out.numpy().reshape(batch, qd)
@@ -347,8 +314,7 @@ def test_attention_prefill_matches_causal_rows(backend, dev):
 @pytest.mark.parametrize("pad", [1, 4])
 def test_attention_prefill_q_stride(backend, dev, orc, pad):
     """Query rows pad floats apart beyond n_heads*head_dim: a stride that
-    16-byte reads cannot follow (pad 1: the rows' scores take the one-row
-    workgroup form) and one they can (pad 4: the multi-row form), each row
+    16-byte reads cannot follow (pad 1) and one they can (pad 4), each row
     bit-exact against the CPU attention."""
     nh, nkv, hd, cap, start, batch = 8, 4, 256, 512, 100, 40
     rng = np.random.default_rng(4700 + pad)

@@ -1,0 +1,69 @@
+"""The dispatch rules of the batched attention and products (csrc/plans.h), CPU only.
+
+The header is compiled for the host, so these tests ask the code itself which
+form a call takes: that the GPU tests' case lists reach every form, and that
+the forms chosen at measured sizes are those measured as the faster ones."""
+
+from __future__ import annotations
+
+import json
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+
+import test_gpu_attention_any as attention_any
+import test_gpu_prefill_ops as prefill_ops
+
+NATIVE = Path(__file__).resolve().parent / "native"
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    """plan(line, ...) -> what plans.h says of each call (plan_dump.cpp)."""
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not available")
+    exe = tmp_path_factory.mktemp("plans") / "plan_dump"
+    subprocess.run(["g++", "-O1", "-std=c++17", str(NATIVE / "plan_dump.cpp"), "-o", str(exe)], check=True)
+
+    def run(lines):
+        out = subprocess.run([str(exe)], input="\n".join(lines), check=True, capture_output=True, text=True).stdout
+        plans = [json.loads(line) for line in out.splitlines()]
+        assert len(plans) == len(lines)
+        return plans
+
+    return run
+
+
+def attn_line(nh, nkv, hd, kf, vf, cap, sw, start, batch):
+    wlimit = sw if sw is not None and 0 < sw < cap else cap
+    return f"attn {start} {batch} {nh} {nkv} {hd} {kf} {vf} {cap} {wlimit}"
+
+
+def prefill_cases():
+    """Every attention_prefill call whose rows the GPU tests compare with the oracle."""
+    yield from attention_any.MANY_ROWS
+    for start, batch, sw, cap, nh, nkv, _ in prefill_ops.PREFILL_CASES:
+        rows = max(1, (64 << 20) // (4 * nh * cap))  # a launch's scores stay within 64 MiB
+        for r0 in range(0, batch, rows):
+            yield nh, nkv, 256, 0, 0, cap, sw, start + r0, min(rows, batch - r0)
+
+
+def test_prefill_cases_reach_every_form(plan):
+    cases = list(prefill_cases())
+    plans = plan([attn_line(*c) for c in cases])
+    scores, softmax, weighted = set(), set(), set()
+    for (nh, nkv, hd, kf, vf, *_), p in zip(cases, plans):
+        scores.add((kf, p["score_m"], min(p["score_reps"], 2)))
+        if p["rows_form"]:
+            chunks = p["span"] > 4 * p["softmax_threads"]
+            softmax.add((p["softmax_threads"], chunks))
+            weighted.add((vf, *p["pv"]))
+        else:
+            weighted.add((vf, "long" if p["long"] else "decode"))
+    assert scores >= {(0, 1, 1), (0, 2, 1), (0, 4, 1), (0, 4, 2), (1, 4, 1), (1, 4, 2), (2, 4, 1), (2, 4, 2)}
+    assert softmax >= {(256, False), (256, True), (512, False), (1024, False), (1024, True)}
+    forms = [(4, 2), (4, 1), (2, 1), (1, 1)]
+    assert weighted >= {(vf, *f) for vf in range(3) for f in forms}
+    assert weighted >= {(vf, f) for vf in range(3) for f in ("decode", "long")}
