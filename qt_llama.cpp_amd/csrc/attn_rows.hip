@@ -57,29 +57,41 @@ __device__ __forceinline__ void scalar_wait()
 }
 
 // ---- scores ------------------------------------------------------------------
-// Workgroup (tile of 64 absolute positions, kv head, block of 4 * M * reps
-// chain rows): the tile's K rows are staged in LDS once (row stride 16 bytes
-// past the data: conflict-free 16-byte reads of 64 rows), then wave w runs
-// chain rows M at a time, lane p the chain of position T0 + p.  Chain row c of
-// a kv head is row c / G, head c % G of the group.  Row blocks are taken in
-// reverse order: the latest rows, with the most tiles, are dispatched first.
-__host__ __device__ constexpr int rows_k_stride(int head_dim) { return head_dim * 2 + 16; }
+// Workgroup (tile of 64 absolute positions that the block's rows can see, kv
+// head, block of 4 * M * reps chain rows): the tile's K rows are staged in LDS
+// once (row stride 16 bytes past the data: conflict-free 16-byte reads of 64
+// rows), then wave w runs chain rows M at a time, lane p the chain of position
+// T0 + p.  Chain row c of a kv head is row c / G, head c % G of the group.  Row
+// blocks are taken in reverse order: the latest rows, with the most tiles, are
+// dispatched first.
+// First position of the workgroup's tile.  all: tile blockIdx.x of the launch's.
+// Otherwise one of the gridDim.x tiles from the one that the block's first
+// row's window (start0) starts in, each at a blockIdx.x that its number alone
+// decides, so that blocks of rows find it in the same XCD's L2 and the workgroups
+// past a block's last position fall to every XCD alike.  (The division is half
+// a microsecond of scalar code, 3 % of a launch of a few rows.)
+__device__ __forceinline__ int block_tile(int all, int start0, int t_lo)
+{
+    if (all) return t_lo + (int)blockIdx.x * kRowsP;
+    const uint32_t n = gridDim.x, first = (uint32_t)(start0 - t_lo) / kRowsP;
+    const int r = (int)blockIdx.x - (int)(first % n);
+    return t_lo + ((int)first + (r < 0 ? r + (int)n : r)) * kRowsP;
+}
 
 template <int M>
 __global__ __launch_bounds__(64 * kRowsW) void attn_rows_scores_kernel(
     const float *__restrict__ q, int q_stride, const uint16_t *__restrict__ k_cache, int n_past0, int nchains,
-    int n_heads, int n_kv_heads, int head_dim, float scale, int capacity, int wlimit, int t_lo, int reps,
-    float *__restrict__ scores)
+    int n_heads, int n_kv_heads, int head_dim, float scale, int capacity, int wlimit, int t_lo, int all_tiles,
+    int reps, float *__restrict__ scores)
 {
     extern __shared__ __align__(16) uint8_t k_s[];
     const int NT = 64 * kRowsW, HD = head_dim, KR = rows_k_stride(HD), G = n_heads / n_kv_heads;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int T0 = t_lo + (int)blockIdx.x * kRowsP, kvh = blockIdx.y;
-    const int per = kRowsW * M * reps, c0 = ((int)gridDim.z - 1 - (int)blockIdx.z) * per;
+    const int kvh = blockIdx.y, per = kRowsW * M * reps, c0 = ((int)gridDim.z - 1 - (int)blockIdx.z) * per;
     const int cl = (c0 + per < nchains ? c0 + per : nchains) - 1;  // the block's last chain row
     int win0, start0;
     attn_window(nullptr, n_past0 + c0 / G, wlimit, win0, start0);
-    const int pos_l = n_past0 + cl / G;
+    const int T0 = block_tile(all_tiles, start0, t_lo), pos_l = n_past0 + cl / G;
     if (T0 > pos_l || start0 - T0 >= kRowsP) return;  // no row of the block has a position in this tile
     // one load a 128-byte line of the block's q rows, so that the scalar loads
     // below find them in this XCD's L2
@@ -91,7 +103,9 @@ __global__ __launch_bounds__(64 * kRowsW) void attn_rows_scores_kernel(
     }
     // K rows: thread -> 16-byte chunk tid % cpr of rows tid / cpr, + rpp, ...
     // Positions past the block's newest one reload that row; their scores are
-    // not stored.  The tile's rows follow the first one's around the ring.
+    // not stored (with a test a load instead, each waits for the one before: 130
+    // us against 124 at 500 rows of 8 x 512 dims).  The tile's rows follow the
+    // first one's around the ring.
     const size_t kv_dim = (size_t)n_kv_heads * HD;
     const uint16_t *kh = k_cache + (size_t)kvh * HD;
     constexpr int kPer = 8;  // rows a thread loads before it stores any
@@ -200,8 +214,8 @@ inline size_t rows_q_lds(int kf, int nb)
 template <int KF>
 __global__ __launch_bounds__(64 * kRowsW) void attn_rows_scores_q_kernel(
     const float *__restrict__ q, int q_stride, const uint8_t *__restrict__ k_cache, int n_past0, int nchains,
-    int n_heads, int n_kv_heads, int nb, float scale, int capacity, int wlimit, int t_lo, int reps,
-    float *__restrict__ scores)
+    int n_heads, int n_kv_heads, int nb, float scale, int capacity, int wlimit, int t_lo, int all_tiles,
+    int reps, float *__restrict__ scores)
 {
     constexpr int M = kRowsQM, NT = 64 * kRowsW, BB = KF == 1 ? 34 : 18, QW = KF == 1 ? 8 : 4;
     extern __shared__ __align__(16) uint32_t q_lds[];
@@ -212,12 +226,11 @@ __global__ __launch_bounds__(64 * kRowsW) void attn_rows_scores_q_kernel(
     float *qd = reinterpret_cast<float *>(qq + kRowsQC * nb * 8);           // [kRowsQC][nb] scales
     int *qs = reinterpret_cast<int *>(qd + kRowsQC * nb);                   // [kRowsQC][nb] quant sums
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int T0 = t_lo + (int)blockIdx.x * kRowsP, kvh = blockIdx.y;
-    const int per = kRowsQC * reps, c0 = ((int)gridDim.z - 1 - (int)blockIdx.z) * per;
+    const int kvh = blockIdx.y, per = kRowsQC * reps, c0 = ((int)gridDim.z - 1 - (int)blockIdx.z) * per;
     const int cl = (c0 + per < nchains ? c0 + per : nchains) - 1;  // the block's last chain row
     int win0, start0;
     attn_window(nullptr, n_past0 + c0 / G, wlimit, win0, start0);
-    const int pos_l = n_past0 + cl / G;
+    const int T0 = block_tile(all_tiles, start0, t_lo), pos_l = n_past0 + cl / G;
     if (T0 > pos_l || start0 - T0 >= kRowsP) return;  // no row of the block has a position in this tile
     {   // four threads a row, blocks tid % 4, + 4, ...
         const int r = tid >> 2, t = T0 + r <= pos_l ? T0 + r : pos_l;
@@ -636,13 +649,14 @@ int launch_attn_rows_scores(mrml_hip_ctx *ctx, const AttnRowsPlan &plan, const f
                             const void *k_cache, int n_past0, int rows, int n_heads, int n_kv_heads, int head_dim,
                             int k_fmt, float scale, int capacity, int wlimit, float *scores)
 {
-    const int nchains = rows * (n_heads / n_kv_heads), t_lo = plan.t_lo, reps = plan.score_reps;
+    const int nchains = rows * (n_heads / n_kv_heads), t_lo = plan.t_lo, reps = plan.score_reps,
+              all = plan.all_tiles;
     const dim3 grid((unsigned)plan.tiles, (unsigned)n_kv_heads, (unsigned)plan.score_blocks(nchains));
     if (k_fmt != 0) {
 #define ROWS_SCQ(KF)                                                                                               \
     hipLaunchKernelGGL(attn_rows_scores_q_kernel<KF>, grid, dim3(64 * kRowsW), rows_q_lds(KF, head_dim / 32),       \
                        ctx->stream, q, q_stride, (const uint8_t *)k_cache, n_past0, nchains, n_heads, n_kv_heads,   \
-                       head_dim / 32, scale, capacity, wlimit, t_lo, reps, scores)
+                       head_dim / 32, scale, capacity, wlimit, t_lo, all, reps, scores)
         if (k_fmt == 1) ROWS_SCQ(1);
         else ROWS_SCQ(2);
 #undef ROWS_SCQ
@@ -652,7 +666,7 @@ int launch_attn_rows_scores(mrml_hip_ctx *ctx, const AttnRowsPlan &plan, const f
 #define ROWS_SC(M)                                                                                               \
     hipLaunchKernelGGL(attn_rows_scores_kernel<M>, grid, dim3(64 * kRowsW), lds, ctx->stream, q, q_stride,          \
                        (const uint16_t *)k_cache, n_past0, nchains, n_heads, n_kv_heads, head_dim, scale, capacity, \
-                       wlimit, t_lo, reps, scores)
+                       wlimit, t_lo, all, reps, scores)
     if (plan.score_m == 4) ROWS_SC(4);
     else if (plan.score_m == 2) ROWS_SC(2);
     else ROWS_SC(1);

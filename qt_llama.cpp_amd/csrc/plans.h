@@ -10,7 +10,7 @@
 
 namespace mrml {
 
-constexpr int kCUs = 256, kSIMDs = 4 * kCUs;  // MI355X
+constexpr int kCUs = 256, kSIMDs = 4 * kCUs, kLdsBytes = 160 << 10;  // MI355X; LDS of a CU
 
 // ---- decode softmax ------------------------------------------------------------
 // The line lies on the widest window of the launch, not on the cache's
@@ -34,15 +34,21 @@ constexpr int kRowsP = 64;    // positions per score tile
 constexpr int kRowsW = 4;     // waves per score workgroup
 constexpr int kRowsQM = 4, kRowsQC = kRowsW * kRowsQM;  // quantised K: chain rows a wave, a pass
 
+#if defined(__HIPCC__)
+__host__ __device__
+#endif
+constexpr int rows_k_stride(int head_dim) { return head_dim * 2 + 16; }  // bytes of a staged f16 K row
+
 struct AttnRowsPlan {
-    int span;        // the widest window
-    int t_lo;        // the first row's window start
-    int tiles;       // score tiles from there to the last row's position
-    int score_m;     // chain rows (row x query head) a wave
-    int score_reps;  // passes over a staged tile
-    bool rows_form;  // softmax and weighted sum as attn_rows.hip has them, else the decode form
+    int span;             // the widest window
+    int t_lo;             // the first row's window start
+    int score_m;          // chain rows (row x query head) a wave
+    int score_reps;       // passes over a staged tile
+    int tiles;            // score tiles dispatched a row block
+    bool all_tiles;       // those are all from t_lo to the last row's position
+    bool rows_form;       // softmax and weighted sum as attn_rows.hip has them, else the decode form
     int softmax_threads;
-    int pv_m, pv_d;  // weighted sum: chain rows a wave, dims a lane
+    int pv_m, pv_d;       // weighted sum: chain rows a wave, dims a lane
     int score_blocks(int nchains) const
     {
         const int per = kRowsW * score_m * score_reps;
@@ -65,21 +71,40 @@ inline AttnRowsPlan attn_rows_plan(int n_past0, int rows, int n_heads, int n_kv_
     p.span = std::min(wlimit, n_past0 + rows);
     // positions tiled absolutely from row 0's window start to the last row's position
     p.t_lo = count0 > wlimit ? count0 - wlimit : 0;
-    p.tiles = (n_past0 + rows - 1 - p.t_lo) / kRowsP + 1;
-    const int64_t chain_tiles = (int64_t)p.tiles * n_kv_heads * nchains;
+    const int tiles = (n_past0 + rows - 1 - p.t_lo) / kRowsP + 1, group = n_heads / n_kv_heads;
+    // the tiles that the chain rows' windows meet: (w + 62) / 64 of w positions on average
+    const int64_t chain_tiles = (int64_t)n_kv_heads * nchains * std::min(tiles * kRowsP, wlimit + kRowsP - 2) / kRowsP;
     if (k_fmt != 0) {
         // passes over a staged tile: as many as leave four workgroups a CU
         p.score_m = kRowsQM;
         p.score_reps = (int)std::min<int64_t>(8, std::max<int64_t>(1, chain_tiles / (kRowsQC * 4 * kCUs)));
     } else {
-        // Chain rows a wave: four while that leaves two waves a SIMD, else two or
-        // one (77 rows of 8 heads at 377 positions: 9.6 us with one, 11 with four).
-        // Two sets of them a workgroup once the launch is many rounds of the chip
-        // (512 rows behind 2048 positions: 10,240 workgroups, 7 us less; 512 rows
-        // from the start: 2048, 2 us more).
-        p.score_m = chain_tiles >= 4 * 2 * kSIMDs ? 4 : (chain_tiles >= 2 * 2 * kSIMDs ? 2 : 1);
+        // Chain rows a wave: one while its workgroups are resident at once (four
+        // a CU, fewer where a tile takes more of the 160 KB of LDS), two up to twice as
+        // many, else four (77 rows of 8 heads at 377 positions: 9.6 us with
+        // one, 11 with four; 80 rows of 8 x 512 dims over one kv head behind
+        // 300 positions, 3840 chain tiles for 2 a CU: 45.5 / 41.6 / 43.4 at 1 / 2 /
+        // 4).  Two sets of them a workgroup once the launch is many rounds of
+        // the chip (512 rows behind 2048 positions: 10,240 workgroups, 7 us
+        // less; 512 rows from the start: 2048, 2 us more).
+        const int64_t resident = (int64_t)kCUs * std::min(4, kLdsBytes / (kRowsP * rows_k_stride(head_dim)));
+        p.score_m = chain_tiles >= 2 * kRowsW * resident ? 4 : (chain_tiles >= kRowsW * resident ? 2 : 1);
         p.score_reps = chain_tiles / (kRowsW * p.score_m) >= 8192 ? 2 : 1;
     }
+    // A row block's tiles: its rows span wlimit positions and one more a row
+    // after the first.  (All tiles of the launch a block left most workgroups
+    // of a sliding window without work: 500 rows x 8 heads over a window of 20
+    // took 48 us, 44 without them.)  With a whole number of rounds of the eight
+    // XCDs over tiles and kv heads, where that adds at most a quarter, a tile
+    // stays on its XCD from block to block (300 rows of 8 heads of 256
+    // dims over a window of 512, Q8_0: 68 us, 70 at 11 tiles instead of 12).
+    const int block_rows = (kRowsW * p.score_m * p.score_reps + group - 2) / group + 1;
+    p.tiles = (wlimit + block_rows - 2) / kRowsP + 2;
+    const int round = n_kv_heads % 8 == 0 ? 1 : n_kv_heads % 4 == 0 ? 2 : n_kv_heads % 2 == 0 ? 4 : 8;
+    const int whole = (p.tiles + round - 1) / round * round;
+    if (4 * whole <= 5 * p.tiles) p.tiles = whole;
+    p.tiles = std::min(tiles, p.tiles);
+    p.all_tiles = p.tiles == tiles;
 
     // The decode form's workgroup adds 32 dims of one row at 4.7 ns a
     // position, the rows form's waves need company for that: while the decode

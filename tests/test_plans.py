@@ -50,6 +50,25 @@ def prefill_cases():
             yield nh, nkv, 256, 0, 0, cap, sw, start + r0, min(rows, batch - r0)
 
 
+def test_score_blocks_dispatch_their_windows(plan):
+    """A row block's tiles hold every position its rows see, and under a sliding
+    window few beyond them (the tiles of the whole launch left most workgroups without work)."""
+    cases = [(nh, nkv, 256, kf, 0, 4096, sw, start, batch)
+             for nh, nkv in ((8, 8), (8, 4), (12, 4), (8, 1)) for kf in (0, 1)
+             for sw in (None, 1, 20, 63, 64, 65, 130, 1000)
+             for start, batch in ((0, 1), (0, 200), (37, 64), (1000, 1), (1000, 500), (3000, 129))]
+    for (nh, nkv, _, kf, _, cap, sw, start, batch), p in zip(cases, plan([attn_line(*c) for c in cases])):
+        g, limit = nh // nkv, sw or cap
+        chains, per = batch * g, 4 * p["score_m"] * p["score_reps"]
+        t_lo = max(0, start + 1 - limit)
+        assert p["score_blocks"] * per >= chains > (p["score_blocks"] - 1) * per
+        for c0 in range(0, chains, per):
+            first, last = start + c0 // g, start + (min(c0 + per, chains) - 1) // g
+            tile0 = t_lo + (max(0, first + 1 - limit) - t_lo) // 64 * 64
+            assert tile0 <= max(0, first + 1 - limit) and tile0 + 64 * p["tiles"] > last
+        assert 4 * 64 * p["tiles"] <= 5 * (limit + per // g + 1 + 3 * 64)
+
+
 def test_prefill_cases_reach_every_form(plan):
     cases = list(prefill_cases())
     plans = plan([attn_line(*c) for c in cases])
