@@ -22,6 +22,8 @@
 
 #include <math.h>
 
+#include <algorithm>
+
 #include "attn_common.h"
 #include "device.h"
 #include "exact_sum.h"
@@ -295,16 +297,11 @@ __global__ __launch_bounds__(512) void attn_scores_kernel(const float *__restric
                                                           const uint16_t *__restrict__ k_cache,
                                                           const int32_t *__restrict__ d_pos, int n_past_arg,
                                                           int n_heads, int n_kv_heads, float scale, int capacity, int wlimit,
-                                                          float *__restrict__ scores, int q_stride)
+                                                          float *__restrict__ scores)
 {
     constexpr int HD = kAttnHD, P = kScoreP;
     __shared__ __align__(16) float q_s[8][HD];
     __shared__ __align__(16) uint8_t k_s[P * kKRow];
-    // query row blockIdx.z of a batch (prefill): rows q_stride floats apart
-    // at consecutive positions
-    q += (size_t)blockIdx.z * q_stride;
-    scores += (size_t)blockIdx.z * n_heads * capacity;
-    n_past_arg += (int)blockIdx.z;
     int window, start;
     attn_window(d_pos, n_past_arg, wlimit, window, start);
     const int p0 = blockIdx.x * P;
@@ -445,7 +442,7 @@ __global__ __launch_bounds__(64) void kv_append_any_kernel(const float *__restri
 // the heads w, w + 4, ... of the group; the K tile is staged through LDS in
 // passes of 128 dims (f16 rows as they are; quantised blocks re-laid as
 // 4-byte-aligned quants plus f32 scales), every chain carried across passes
-// in registers.  Dynamic LDS as attn_any_scores_lds says.
+// in registers.  Grid z: query rows of a batch.  Dynamic LDS as attn_any_scores_lds says.
 constexpr int kAnyP = 64;                   // positions per workgroup (one per lane)
 constexpr int kAnyT = 256;                  // 4 waves
 constexpr int kAnyCh = 128;                 // dims per pass (4 blocks)
@@ -467,9 +464,14 @@ __global__ __launch_bounds__(kAnyT) void attn_scores_any_kernel(const float *__r
                                                                 const uint8_t *__restrict__ k_cache,
                                                                 const int32_t *__restrict__ d_pos, int n_past_arg,
                                                                 int n_heads, int n_kv_heads, int head_dim, float scale,
-                                                                int capacity, int wlimit, float *__restrict__ scores)
+                                                                int capacity, int wlimit, float *__restrict__ scores,
+                                                                int q_stride)
 {
     extern __shared__ __align__(16) uint8_t lds_any[];
+    // query row blockIdx.z of a batch: rows q_stride floats apart at consecutive positions
+    q += (size_t)blockIdx.z * q_stride;
+    scores += (size_t)blockIdx.z * n_heads * capacity;
+    n_past_arg += (int)blockIdx.z;
     int window, start;
     attn_window(d_pos, n_past_arg, wlimit, window, start);
     const int p0 = blockIdx.x * kAnyP;
@@ -1583,23 +1585,52 @@ static int launch_softmax_v(mrml_hip_ctx *ctx, const float *scores, const void *
     return check_launch(ctx, "attn_softmax_v_kernel");
 }
 
+// Scores of `rows` query rows, a workgroup a row, kv head and tile of 64
+// positions of its window (every tile when the position is on the device).
+// tuned: the kernels for f16 rows of 256 dims and groups of up to 8 (batches:
+// up to 4).
+static int launch_decode_scores(mrml_hip_ctx *ctx, const float *q, int q_stride, const void *k_cache,
+                                const int32_t *d_pos, int n_past, int rows, int n_heads, int n_kv_heads, int head_dim,
+                                int k_fmt, bool tuned, float scale, int capacity, int wlimit, float *scores)
+{
+    const int G = n_heads / n_kv_heads;
+    const dim3 grid((attn_span(d_pos, n_past, rows, wlimit) + kScoreP - 1) / kScoreP, n_kv_heads, rows);
+    uint16_t *k16 = const_cast<uint16_t *>(reinterpret_cast<const uint16_t *>(k_cache));
+    if (tuned && G <= 4) {
+        hipLaunchKernelGGL(attn_scores2_kernel<false>, grid, dim3(kScoreT), 0, ctx->stream, q, k16,
+                           (uint16_t *)nullptr, d_pos, n_past, n_heads, n_kv_heads, scale, capacity, wlimit,
+                           RopeArgs{}, scores, q_stride);
+        return check_launch(ctx, "attn_scores2_kernel");
+    }
+    if (tuned) {
+        hipLaunchKernelGGL(attn_scores_kernel, grid, dim3(64 * G), 0, ctx->stream, q, k16, d_pos, n_past, n_heads,
+                           n_kv_heads, scale, capacity, wlimit, scores);
+        return check_launch(ctx, "attn_scores_kernel");
+    }
+    const size_t lds = attn_any_scores_lds(k_fmt, G, head_dim);
+    const uint8_t *kc = reinterpret_cast<const uint8_t *>(k_cache);
+#define SC_LAUNCH(KF)                                                                                             \
+    hipLaunchKernelGGL(attn_scores_any_kernel<KF>, grid, dim3(kAnyT), lds, ctx->stream, q, kc, d_pos, n_past,     \
+                       n_heads, n_kv_heads, head_dim, scale, capacity, wlimit, scores, q_stride)
+    if (k_fmt == 1)
+        SC_LAUNCH(1);
+    else if (k_fmt == 2)
+        SC_LAUNCH(2);
+    else
+        SC_LAUNCH(0);
+#undef SC_LAUNCH
+    return check_launch(ctx, "attn_scores_any_kernel");
+}
+
 int launch_attn_decode_f16(mrml_hip_ctx *ctx, const float *q, const uint16_t *k_cache, const uint16_t *v_cache,
                            float *out, void *pack, const int32_t *d_pos, int n_past, int n_heads, int n_kv_heads,
                            float scale, int capacity, void *scratch, int sliding_window)
 {
     float *scores = reinterpret_cast<float *>(scratch);
     const int wlimit = attn_window_limit(capacity, sliding_window);
-    const dim3 sgrid((attn_span(d_pos, n_past, 1, wlimit) + kScoreP - 1) / kScoreP, n_kv_heads);
-    if (n_heads / n_kv_heads <= 4) {
-        hipLaunchKernelGGL(attn_scores2_kernel<false>, sgrid, dim3(kScoreT), 0, ctx->stream, q,
-                           const_cast<uint16_t *>(k_cache), (uint16_t *)nullptr, d_pos, n_past, n_heads, n_kv_heads,
-                           scale, capacity, wlimit, RopeArgs{}, scores, 0);
-        if (int rc = check_launch(ctx, "attn_scores2_kernel")) return rc;
-    } else {
-        hipLaunchKernelGGL(attn_scores_kernel, sgrid, dim3(64 * (n_heads / n_kv_heads)), 0, ctx->stream, q, k_cache,
-                           d_pos, n_past, n_heads, n_kv_heads, scale, capacity, wlimit, scores, 0);
-        if (int rc = check_launch(ctx, "attn_scores_kernel")) return rc;
-    }
+    if (int rc = launch_decode_scores(ctx, q, 0, k_cache, d_pos, n_past, 1, n_heads, n_kv_heads, kAttnHD, 0, true,
+                                      scale, capacity, wlimit, scores))
+        return rc;
     return launch_softmax_v(ctx, scores, v_cache, out, pack, d_pos, n_past, n_heads, n_kv_heads, capacity, wlimit);
 }
 
@@ -1641,21 +1672,9 @@ int launch_attn_any(mrml_hip_ctx *ctx, const float *q, const void *k_cache, cons
 {
     float *scores = reinterpret_cast<float *>(scratch);
     const int wlimit = attn_window_limit(capacity, sliding_window);
-    // score tiles up to the window (every tile when the position is on the device)
-    const dim3 sgrid((attn_span(d_pos, n_past, 1, wlimit) + kAnyP - 1) / kAnyP, n_kv_heads);
-    const size_t lds = attn_any_scores_lds(k_fmt, n_heads / n_kv_heads, head_dim);
-    const uint8_t *kc = reinterpret_cast<const uint8_t *>(k_cache);
-#define SC_LAUNCH(KF)                                                                                             \
-    hipLaunchKernelGGL(attn_scores_any_kernel<KF>, sgrid, dim3(kAnyT), lds, ctx->stream, q, kc, d_pos, n_past,    \
-                       n_heads, n_kv_heads, head_dim, scale, capacity, wlimit, scores)
-    if (k_fmt == 1)
-        SC_LAUNCH(1);
-    else if (k_fmt == 2)
-        SC_LAUNCH(2);
-    else
-        SC_LAUNCH(0);
-#undef SC_LAUNCH
-    if (int rc = check_launch(ctx, "attn_scores_any_kernel")) return rc;
+    if (int rc = launch_decode_scores(ctx, q, 0, k_cache, d_pos, n_past, 1, n_heads, n_kv_heads, head_dim, k_fmt, false,
+                                      scale, capacity, wlimit, scores))
+        return rc;
     return launch_softmax_v(ctx, scores, v_cache, out, pack, d_pos, n_past, n_heads, n_kv_heads, capacity, wlimit, 1,
                             head_dim, v_fmt);
 }
@@ -1673,9 +1692,13 @@ int launch_attn_rows(mrml_hip_ctx *ctx, const float *q, int q_stride, const void
     float *scores = reinterpret_cast<float *>(scratch);
     const int wlimit = attn_window_limit(capacity, sliding_window);
     const AttnRowsPlan plan = attn_rows_plan(n_past0, rows, n_heads, n_kv_heads, head_dim, k_fmt, v_fmt, capacity, wlimit);
-    if (int rc = launch_attn_rows_scores(ctx, plan, q, q_stride, k_cache, n_past0, rows, n_heads, n_kv_heads, head_dim,
-                                         k_fmt, scale, capacity, wlimit, scores))
-        return rc;
+    const int rc = plan.one_row_scores
+                       ? launch_decode_scores(ctx, q, q_stride, k_cache, nullptr, n_past0, rows, n_heads, n_kv_heads,
+                                              head_dim, k_fmt, head_dim == kAttnHD && k_fmt == 0, scale, capacity,
+                                              wlimit, scores)
+                       : launch_attn_rows_scores(ctx, plan, q, q_stride, k_cache, n_past0, rows, n_heads, n_kv_heads,
+                                                 head_dim, k_fmt, scale, capacity, wlimit, scores);
+    if (rc) return rc;
     if (!plan.rows_form)
         return launch_softmax_v(ctx, scores, v_cache, out, nullptr, nullptr, n_past0, n_heads, n_kv_heads, capacity,
                                 wlimit, rows, head_dim, v_fmt);

@@ -42,6 +42,7 @@ constexpr int rows_k_stride(int head_dim) { return head_dim * 2 + 16; }  // byte
 struct AttnRowsPlan {
     int span;             // the widest window
     int t_lo;             // the first row's window start
+    bool one_row_scores;  // scores by the decode kernels, a workgroup a row, else by attn_rows.hip's:
     int score_m;          // chain rows (row x query head) a wave
     int score_reps;       // passes over a staged tile
     int tiles;            // score tiles dispatched a row block
@@ -105,6 +106,24 @@ inline AttnRowsPlan attn_rows_plan(int n_past0, int rows, int n_heads, int n_kv_
     if (4 * whole <= 5 * p.tiles) p.tiles = whole;
     p.tiles = std::min(tiles, p.tiles);
     p.all_tiles = p.tiles == tiles;
+
+    // Few rows: the decode kernels, which take a workgroup a row, kv head and
+    // tile and have q in LDS, are done before attn_rows_scores_kernel at one
+    // chain row a wave, whose scalar loads of q are waited for one after another
+    // (whole attention, 8 / 4 heads of 256 dims: 16 rows at 100 positions 16.3 us
+    // against 17.9, 1 row at 2500 26.5 against 27.8; 8 x 64 dims, 8 rows from 0
+    // 11.1 / 11.6), up to four of these workgroups a CU (16 rows of 8 kv heads at 700,
+    // 1536 of them: 39.3 / 37.9; 64 of 4 at 100, 768: 20.1 / 21.0; 128 of 4 from
+    // 0, 1024: equal).  Not for groups past four heads (two heads a wave there:
+    // 16 / 2 heads of 128 14.1 / 12.8), 96 to 224 dims (8 of 128: 12.6 / 12.6)
+    // or more (groups of 8 heads of 512: 25.4 / 16.9), quantised K (8 / 4 heads of
+    // 256, Q8_0: 18.7 / 15.3), or windows whose last tile holds eight positions
+    // or fewer, where a workgroup loads the last row for all of the others (4 /
+    // 1 heads at a window of 200, 40 rows: 21.3 / 20.8; 8 / 8 heads 26.2 / 25.0).
+    const int64_t one_row = (int64_t)((p.span + kRowsP - 1) / kRowsP) * n_kv_heads * rows;
+    const int window0 = std::min(wlimit, count0);
+    const bool thin = (window0 - 1) % kRowsP < 8 && (group == 4 || (window0 == wlimit && rows > 8));
+    p.one_row_scores = k_fmt == 0 && group <= 4 && (head_dim == 256 || head_dim <= 64) && one_row <= 4 * kCUs && !thin;
 
     // The decode form's workgroup adds 32 dims of one row at 4.7 ns a
     // position, the rows form's waves need company for that: while the decode

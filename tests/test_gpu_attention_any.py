@@ -240,6 +240,9 @@ MANY_ROWS = [
     (8, 4, 256, 0, 0, 8192, None, 5000, 20),   # softmax in chunks of 1024 threads
     (8, 4, 256, 1, 1, 512, None, 300, 6),      # decode form over quantised rows
     (8, 2, 128, 2, 2, 512, 130, 300, 12),
+    (8, 8, 64, 0, 0, 300, 90, 280, 21),        # scores a workgroup a row: any head size, the ring's end inside
+    (9, 3, 32, 0, 0, 128, None, 0, 70),
+    (6, 2, 256, 0, 0, 200, 70, 190, 40),       # and 256 dims, group of 3
     # the long softmax with several rows, at every value format; the second and third across whole chunks
     (4, 2, 64, 0, 0, 16384, None, 11000, 3),
     (4, 2, 64, 1, 1, 16384, None, 16380, 4),
@@ -257,7 +260,7 @@ def test_attention_prefill_many_rows(backend, dev, orc, nh, nkv, hd, kf, vf, cap
         # outside the earliest row's window: the row must not meet it (0 * inf)
         vx[(start + batch - 1) % cap, 0] = np.inf
     kc, vc = cache_bytes(orc, kx, kf), cache_bytes(orc, vx, vf)
-    stride = qd + 2 * kvd + (1 if hd == 96 else 0)  # q rows off 16 bytes too
+    stride = qd + 2 * kvd + (1 if hd == 96 or nh == 9 else 0)  # q rows off 16 bytes too
     q = (rng.standard_normal(batch * stride) * 0.5).astype(np.float32)
     qb, kb, vb = backend.HipBuffer.from_host(dev, q), upload_cache(backend, dev, kc), upload_cache(backend, dev, vc)
     out = backend.HipBuffer.alloc(dev, batch * qd)

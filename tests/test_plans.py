@@ -69,18 +69,38 @@ def test_score_blocks_dispatch_their_windows(plan):
         assert 4 * 64 * p["tiles"] <= 5 * (limit + per // g + 1 + 3 * 64)
 
 
+# (heads, kv heads, dims, K format, start, batch): where the decode kernels' scores measured
+# faster, and where not
+ONE_ROW = [(8, 4, 256, 0, 100, 16), (8, 8, 256, 0, 0, 64), (4, 4, 256, 0, 700, 8), (16, 4, 256, 0, 40, 8),
+           (8, 8, 64, 0, 0, 8), (2, 2, 32, 0, 700, 3), (32, 8, 64, 0, 100, 3)]
+NOT_ONE_ROW = [(8, 4, 256, 0, 700, 32), (8, 8, 256, 0, 100, 64), (16, 4, 256, 0, 0, 4), (8, 1, 256, 0, 0, 8),
+               (8, 1, 512, 0, 0, 3), (8, 4, 256, 1, 0, 3), (8, 8, 64, 0, 2500, 16)]
+
+
+def test_few_rows_take_the_decode_scores(plan):
+    for cases, want in ((ONE_ROW, 1), (NOT_ONE_ROW, 0)):
+        lines = [attn_line(nh, nkv, hd, kf, 0, 4096, None, start, batch) for nh, nkv, hd, kf, start, batch in cases]
+        assert [p["one_row_scores"] for p in plan(lines)] == [want] * len(cases)
+    windows = [attn_line(8, 8, 256, 0, 0, 4096, w, 1000, 20) for w in (64, 65, 72, 73, 200, 208)]
+    assert [p["one_row_scores"] for p in plan(windows)] == [1, 0, 0, 1, 0, 1]
+
+
 def test_prefill_cases_reach_every_form(plan):
     cases = list(prefill_cases())
     plans = plan([attn_line(*c) for c in cases])
     scores, softmax, weighted = set(), set(), set()
     for (nh, nkv, hd, kf, vf, *_), p in zip(cases, plans):
-        scores.add((kf, p["score_m"], min(p["score_reps"], 2)))
+        if p["one_row_scores"]:
+            scores.add("tuned" if hd == 256 else "any")
+        else:
+            scores.add((kf, p["score_m"], min(p["score_reps"], 2)))
         if p["rows_form"]:
             chunks = p["span"] > 4 * p["softmax_threads"]
             softmax.add((p["softmax_threads"], chunks))
             weighted.add((vf, *p["pv"]))
         else:
             weighted.add((vf, "long" if p["long"] else "decode"))
+    assert scores >= {"tuned", "any"}
     assert scores >= {(0, 1, 1), (0, 2, 1), (0, 4, 1), (0, 4, 2), (1, 4, 1), (1, 4, 2), (2, 4, 1), (2, 4, 2)}
     assert softmax >= {(256, False), (256, True), (512, False), (1024, False), (1024, True)}
     forms = [(4, 2), (4, 1), (2, 1), (1, 1)]
