@@ -684,7 +684,8 @@ int launch_attn_rows_softmax_v(mrml_hip_ctx *ctx, const AttnRowsPlan &plan, floa
 #define ROWS_SM(NT)                                                                                              \
     hipLaunchKernelGGL(attn_rows_softmax_kernel<NT>, sgrid, dim3(NT), 0, ctx->stream, scores, n_past0, n_heads,   \
                        capacity, wlimit, fe)
-    if (nt == 256) ROWS_SM(256);
+    if (nt == 64) ROWS_SM(64);
+    else if (nt == 256) ROWS_SM(256);
     else if (nt == 512) ROWS_SM(512);
     else ROWS_SM(1024);
 #undef ROWS_SM
@@ -699,10 +700,10 @@ int launch_attn_rows_softmax_v(mrml_hip_ctx *ctx, const AttnRowsPlan &plan, floa
         hipLaunchKernelGGL((attn_rows_pv_kernel<VF, M, D>), dim3(wgs), dim3(256), 0, ctx->stream, scores, v,       \
                            n_past0, nchains, n_heads, n_kv_heads, head_dim, capacity, wlimit, nblk, nsl, out);     \
     } while (0)
-#define ROWS_PV_MD(VF)                                                                                             \
+#define ROWS_PV_MD(VF)  /* (4 x 1 over Q8_0: never chosen, not built) */                                           \
     do {                                                                                                           \
-        if (plan.pv_m == 4 && plan.pv_d == 2) ROWS_PV(VF, 4, 2);                                                   \
-        else if (plan.pv_m == 4) ROWS_PV(VF, 4, 1);                                                                \
+        if (plan.pv_m == 4 && (VF == 1 || plan.pv_d == 2)) ROWS_PV(VF, 4, 2);                                      \
+        else if (plan.pv_m == 4) ROWS_PV(VF, 4, (VF == 1 ? 2 : 1));                                                \
         else if (plan.pv_m == 2) ROWS_PV(VF, 2, 1);                                                                \
         else ROWS_PV(VF, 1, 1);                                                                                    \
     } while (0)

@@ -118,11 +118,12 @@ inline AttnRowsPlan attn_rows_plan(int n_past0, int rows, int n_heads, int n_kv_
     // 16 / 2 heads of 128 14.1 / 12.8), 96 to 224 dims (8 of 128: 12.6 / 12.6)
     // or more (groups of 8 heads of 512: 25.4 / 16.9), quantised K (8 / 4 heads of
     // 256, Q8_0: 18.7 / 15.3), or windows whose last tile holds eight positions
-    // or fewer, where a workgroup loads the last row for all of the others (4 /
-    // 1 heads at a window of 200, 40 rows: 21.3 / 20.8; 8 / 8 heads 26.2 / 25.0).
+    // or fewer, where a workgroup of the 256-dim kernel loads the last row for all
+    // of the others (4 / 1 heads at a window of 200, 40 rows: 21.3 / 20.8; 8 / 8
+    // heads 26.2 / 25.0; 8 / 8 heads of 64, 10 rows: 12.2 / 12.9).
     const int64_t one_row = (int64_t)((p.span + kRowsP - 1) / kRowsP) * n_kv_heads * rows;
     const int window0 = std::min(wlimit, count0);
-    const bool thin = (window0 - 1) % kRowsP < 8 && (group == 4 || (window0 == wlimit && rows > 8));
+    const bool thin = head_dim == 256 && (window0 - 1) % kRowsP < 8 && (group == 4 || (window0 == wlimit && rows > 8));
     p.one_row_scores = k_fmt == 0 && group <= 4 && (head_dim == 256 || head_dim <= 64) && one_row <= 4 * kCUs && !thin;
 
     // The decode form's workgroup adds 32 dims of one row at 4.7 ns a
@@ -137,27 +138,46 @@ inline AttnRowsPlan attn_rows_plan(int n_past0, int rows, int n_heads, int n_kv_
     p.rows_form = !(wgs <= 512 || (wgs <= 1024 && p.span > 512)) &&
                   attn_rows_v_ok(n_kv_heads, head_dim, v_fmt, capacity);
 
+    // Windows up to 256 positions: one wave a row and head, no barrier to wait
+    // at (200 rows x 8 heads, window 20: 29.7 us, 27.3 with it, whole attention).
     // Rows enough to fill the chip: small workgroups, more of them a CU, and
     // chunks past 1024 positions (512 rows x 8 heads of 2300 positions: 54 us,
     // 65 with 512 threads, 76 with 1024).  Few rows: the latency of one chunk
     // counts (4 rows of 3000 positions: 6 us with 1024 threads, 13 with 256).
-    p.softmax_threads = p.span <= 1024 || (int64_t)rows * n_heads >= 1024 ? 256 : (p.span <= 2048 ? 512 : 1024);
+    p.softmax_threads = p.span <= 256 ? 64
+                        : p.span <= 1024 || (int64_t)rows * n_heads >= 1024 ? 256
+                        : p.span <= 2048 ? 512 : 1024;
 
-    // The widest form that leaves waves enough: the four-row forms issue the
-    // fewest conversions and loads a product, the narrow ones keep more SIMDs
-    // busy.  us at (4,2) / (4,1) / (2,1) / (1,1), whole attention, waves of the
-    // first: 512 rows behind 2048 (2048) 347 / 364 / 490 / 741; 333 rows from
-    // 0 (1332) 46.3 / 43.5 / 47.3 / 61; 77 rows behind 300 (308) 37.6 / 32.6 /
-    // 31.3 / 36.2; 200 rows of 4 x 64 dims, window 512 (200) 46 / 40 / 33 / 29.
-    // Quantised rows cost more a load: 300 rows of 8 x 128 Q8_0 (600) 196 /
-    // 233 / 223 / 292.
+    // Weighted sum: the four-row forms issue the fewest conversions and loads a
+    // product, the narrow ones keep more SIMDs busy, so a form is left once it
+    // has more than about one wave a SIMD (1024).  us at (4,2) / (4,1) / (2,1) /
+    // (1,1), whole attention:
+    //   f16, 256 dims: 1280 waves of (1,1) behind 2500 positions 149 / 115 / 99 / 120,
+    //     1024 behind 700 - / - / 35.5 / 34.4; 1200 of (4,1) 211 / 177 / 203 / 273,
+    //     640 38.2 / 33.3 / 32.8 / 37.5; (4,2) is level with (4,1) at 2000 waves of
+    //     its own (behind 0 / 300 / 2500 positions: 79 / 76, 105 / 104, 384 / 405);
+    //   Q8_0, where a lane's one dim is a byte load: (4,1) is never the best,
+    //     (4,2) is from 400 (behind 300, 320: 42.4 / 50.8 / 42.1 / 53.0, 600: 52 / 64 /
+    //     60 / 84);
+    //   Q4_0: (4,1) from 512 (640: 45.1 / 38.3 / 42.3 / 53.1, 320: 41.6 / 35.5 / 32.3
+    //     / 41.5); (4,2), a byte a lane, from 1000 where a head is two of its
+    //     slices (1200 behind 2500: 340 / 376), later where it is one (16 / 4
+    //     heads of 128, 2000: 178 / 167).
+    // A lane of two dims needs 128 of them, but for Q8_0.  Windows up to 160
+    // positions are mostly their ends, which few rows share: two rows a wave (200
+    // rows, window 20, 24.4 at (4,1), 21.1; 150 from 0 over Q8_0 29.1 at (4,2),
+    // 27.6), up to 1536 waves of (4,2) (window 100, Q8_0, 1200 41.2 / 42.8, 2000
+    // 51.2 / 53.7).
     auto waves = [&](int m, int d) {
         return (int64_t)n_kv_heads * ((nchains + m - 1) / m) * ((head_dim + 64 * d - 1) / (64 * d));
     };
+    const bool ends = p.span <= 160, lanes2 = head_dim > 64 || v_fmt == 1;
+    const int min42 = ends ? 1536 : v_fmt == 0 ? 2 * kSIMDs : v_fmt == 1 ? 400 : head_dim >= 256 ? 1000 : 2400;
+    const int min41 = v_fmt == 0 ? kSIMDs : kSIMDs / 2;
     p.pv_m = 1, p.pv_d = 1;
-    if (waves(4, 2) >= (v_fmt == 0 ? 2048 : 600)) p.pv_m = 4, p.pv_d = 2;
-    else if (waves(4, 1) >= 800) p.pv_m = 4;
-    else if (waves(2, 1) >= 800) p.pv_m = 2;
+    if (lanes2 && waves(4, 2) >= min42) p.pv_m = 4, p.pv_d = 2;
+    else if (v_fmt != 1 && !ends && waves(4, 1) >= min41) p.pv_m = 4;
+    else if (waves(1, 1) > kSIMDs) p.pv_m = 2;
     return p;
 }
 

@@ -210,33 +210,34 @@ def test_attention_prefill_any(backend, dev, orc, nh, nkv, hd, kf, vf):
 
 
 # Batches that take the many-row kernels (attn_rows.hip), by what can go wrong
-# there: each weighted-sum form (chain rows x dims a wave: 4x2, 4x1, 2x1, 1x1)
-# at every value format, groups of 3, head sizes whose last 64-dim slice is
+# there (test_plans.py: which forms they reach): each weighted-sum form at
+# every value format, groups of 3, head sizes whose last 64-dim slice is
 # ragged, rows whose windows start or end apart (sliding windows, a window of
 # one position), the ring's end inside the window, capacities below a tile,
 # softmax rows of one chunk and of several (1024 rows x heads and more past
 # 1024 positions), and the decode form's side of the line.
 MANY_ROWS = [
-    (8, 4, 256, 0, 0, 1024, None, 300, 300),   # 4x1, tail batches of every length
-    (8, 4, 256, 0, 0, 2048, None, 0, 513),     # 4x2, from position 0
-    (8, 4, 256, 0, 0, 256, None, 500, 77),     # 2x1, the ring wrapped
+    (8, 4, 256, 0, 0, 1024, None, 300, 300),   # tail batches of every length
+    (8, 4, 256, 0, 0, 2048, None, 0, 513),     # from position 0
+    (8, 4, 256, 0, 0, 256, None, 500, 77),     # the ring wrapped
     (16, 2, 128, 0, 0, 4096, None, 1030, 70),  # softmax in chunks
     (12, 4, 96, 0, 0, 512, 100, 290, 200),     # group of 3, ragged slice, sliding
     (4, 4, 64, 0, 0, 512, 1, 40, 300),         # one position a window
     (4, 4, 32, 0, 0, 40, 7, 100, 300),         # a capacity below a tile
     (8, 1, 512, 0, 0, 640, 333, 400, 90),      # group of 8, 512 dims
-    (8, 4, 256, 1, 2, 512, 200, 450, 150),     # quantised, 4x2, the ring's end inside
+    (8, 4, 256, 1, 2, 512, 200, 450, 150),     # quantised, the ring's end inside
     (8, 2, 128, 2, 1, 512, None, 200, 150),
-    (4, 4, 64, 1, 1, 256, 50, 100, 170),       # quantised, 1x1
-    (6, 2, 96, 2, 2, 300, 130, 280, 130),      # 2x1
+    (4, 4, 64, 1, 1, 256, 50, 100, 170),
+    (6, 2, 96, 2, 2, 300, 130, 280, 130),
     (8, 4, 256, 0, 0, 512, None, 100, 8),      # decode form (512 workgroups)
     (8, 4, 256, 0, 0, 512, None, 100, 9),
     (8, 4, 256, 0, 0, 4096, None, 2048, 512),  # two passes over a staged score tile
-    (8, 4, 256, 1, 1, 1024, None, 100, 460),   # the same over quantised K; Q8_0 at 4x2
+    (8, 4, 256, 1, 1, 1024, None, 100, 460),   # the same over quantised K
     (8, 4, 256, 2, 2, 1024, None, 100, 460),
-    (8, 4, 256, 2, 1, 512, None, 200, 120),    # Q8_0 at 4x1
-    (8, 4, 256, 1, 2, 512, None, 200, 110),    # Q4_0 at 4x1
-    (8, 2, 128, 1, 2, 512, 100, 200, 140),     # Q4_0 at 2x1
+    (8, 4, 256, 2, 1, 512, None, 200, 120),
+    (8, 4, 256, 1, 2, 512, None, 200, 110),
+    (8, 2, 128, 1, 2, 512, 100, 200, 140),
+    (4, 4, 64, 1, 2, 256, 50, 100, 150),
     (8, 4, 256, 0, 0, 8192, None, 5000, 20),   # softmax in chunks of 1024 threads
     (8, 4, 256, 1, 1, 512, None, 300, 6),      # decode form over quantised rows
     (8, 2, 128, 2, 2, 512, 130, 300, 12),

@@ -83,6 +83,24 @@ def test_few_rows_take_the_decode_scores(plan):
         assert [p["one_row_scores"] for p in plan(lines)] == [want] * len(cases)
     windows = [attn_line(8, 8, 256, 0, 0, 4096, w, 1000, 20) for w in (64, 65, 72, 73, 200, 208)]
     assert [p["one_row_scores"] for p in plan(windows)] == [1, 0, 0, 1, 0, 1]
+    assert plan([attn_line(8, 8, 64, 0, 0, 4096, 200, 1000, 10)])[0]["one_row_scores"] == 1
+
+
+# (heads, kv heads, dims, V format, window, start, batch) -> chain rows a wave x dims a lane of the weighted sum,
+# measured the fastest of the four there
+PV = {(8, 4, 256, 0, None, 2500, 40): [2, 1], (8, 4, 256, 0, None, 2500, 80): [2, 1],
+      (8, 4, 256, 0, None, 2500, 150): [4, 1], (4, 4, 256, 0, None, 950, 64): [1, 1],
+      (8, 1, 512, 0, None, 2500, 300): [4, 2], (8, 8, 64, 0, None, 300, 500): [2, 1],
+      (8, 4, 256, 0, 20, 1000, 200): [2, 1], (8, 4, 256, 1, None, 2500, 40): [2, 1],
+      (8, 4, 256, 1, None, 2500, 150): [4, 2], (8, 2, 128, 1, None, 2500, 80): [2, 1],
+      (8, 4, 256, 2, None, 2500, 40): [2, 1], (8, 4, 256, 2, None, 2500, 80): [4, 1],
+      (8, 4, 256, 2, None, 2500, 300): [4, 2], (16, 4, 128, 2, None, 2500, 300): [4, 1],
+      (8, 8, 64, 2, None, 2500, 80): [1, 1], (8, 8, 64, 2, None, 2500, 300): [4, 1]}
+
+
+def test_weighted_sum_form(plan):
+    got = plan([attn_line(nh, nkv, hd, vf, vf, 4096, sw, start, batch) for nh, nkv, hd, vf, sw, start, batch in PV])
+    assert [p["pv"] for p in got] == list(PV.values())
 
 
 def test_prefill_cases_reach_every_form(plan):
@@ -102,7 +120,7 @@ def test_prefill_cases_reach_every_form(plan):
             weighted.add((vf, "long" if p["long"] else "decode"))
     assert scores >= {"tuned", "any"}
     assert scores >= {(0, 1, 1), (0, 2, 1), (0, 4, 1), (0, 4, 2), (1, 4, 1), (1, 4, 2), (2, 4, 1), (2, 4, 2)}
-    assert softmax >= {(256, False), (256, True), (512, False), (1024, False), (1024, True)}
+    assert softmax >= {(64, False), (256, False), (256, True), (512, False), (1024, False), (1024, True)}
     forms = [(4, 2), (4, 1), (2, 1), (1, 1)]
-    assert weighted >= {(vf, *f) for vf in range(3) for f in forms}
+    assert weighted >= {(vf, *f) for vf in range(3) for f in forms if (vf, f) != (1, (4, 1))}  # (not built)
     assert weighted >= {(vf, f) for vf in range(3) for f in ("decode", "long")}
