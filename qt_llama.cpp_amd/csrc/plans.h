@@ -88,8 +88,11 @@ inline AttnRowsPlan attn_rows_plan(int n_past0, int rows, int n_heads, int n_kv_
         // 4).  Two sets of them a workgroup once the launch is many rounds of
         // the chip (512 rows behind 2048 positions: 10,240 workgroups, 7 us
         // less; 512 rows from the start: 2048, 2 us more).
+        // (Past 256 dims a quarter later: 2176 chain tiles of 512 dims 42.1 / 44.3, 2880
+        // 45.7 / 42.5.)
         const int64_t resident = (int64_t)kCUs * std::min(4, kLdsBytes / (kRowsP * rows_k_stride(head_dim)));
-        p.score_m = chain_tiles >= 2 * kRowsW * resident ? 4 : (chain_tiles >= kRowsW * resident ? 2 : 1);
+        const int64_t one = kRowsW * resident * (head_dim > 256 ? 5 : 4) / 4;
+        p.score_m = chain_tiles >= 2 * one ? 4 : (chain_tiles >= one ? 2 : 1);
         p.score_reps = chain_tiles / (kRowsW * p.score_m) >= 8192 ? 2 : 1;
     }
     // A row block's tiles: its rows span wlimit positions and one more a row
@@ -114,7 +117,8 @@ inline AttnRowsPlan attn_rows_plan(int n_past0, int rows, int n_heads, int n_kv_
     // against 17.9, 1 row at 2500 26.5 against 27.8; 8 x 64 dims, 8 rows from 0
     // 11.1 / 11.6), up to four of these workgroups a CU (16 rows of 8 kv heads at 700,
     // 1536 of them: 39.3 / 37.9; 64 of 4 at 100, 768: 20.1 / 21.0; 128 of 4 from
-    // 0, 1024: equal).  Not for groups past four heads (two heads a wave there:
+    // 0, 1024: equal), eight for groups of four (16 / 4 heads, 1280: 86.8 / 87.9, 2560
+    // level; 32 / 8 of 64 dims, 2560: 48.3 / 49.1).  Not for groups past four heads (two heads a wave there:
     // 16 / 2 heads of 128 14.1 / 12.8), 96 to 224 dims (8 of 128: 12.6 / 12.6)
     // or more (groups of 8 heads of 512: 25.4 / 16.9), quantised K (8 / 4 heads of
     // 256, Q8_0: 18.7 / 15.3), or windows whose last tile holds eight positions
@@ -124,19 +128,31 @@ inline AttnRowsPlan attn_rows_plan(int n_past0, int rows, int n_heads, int n_kv_
     const int64_t one_row = (int64_t)((p.span + kRowsP - 1) / kRowsP) * n_kv_heads * rows;
     const int window0 = std::min(wlimit, count0);
     const bool thin = head_dim == 256 && (window0 - 1) % kRowsP < 8 && (group == 4 || (window0 == wlimit && rows > 8));
-    p.one_row_scores = k_fmt == 0 && group <= 4 && (head_dim == 256 || head_dim <= 64) && one_row <= 4 * kCUs && !thin;
+    p.one_row_scores = k_fmt == 0 && group <= 4 && (head_dim == 256 || head_dim <= 64) &&
+                       one_row <= std::max(4, 2 * group) * kCUs && !thin;
 
-    // The decode form's workgroup adds 32 dims of one row at 4.7 ns a
-    // position, the rows form's waves need company for that: while the decode
-    // form's workgroups are all resident at once (three or four a CU) and its
-    // repeated softmax is not what they spend their time on, it is the faster.
-    // Measured (us, decode form / rows form, 8 heads): 8 rows x 256 dims (512
-    // workgroups) at 300 positions 20 / 22, at 3000 75 / 83; 12 rows (768) at
-    // 300 25 / 22; 60 rows x 64 dims (960) at 1000 54 / 66; 20 rows x 256
-    // (1280) at 512 47 / 44; 32 rows (2048) at 100 44 / 19.
+    // The decode form's workgroups (32 dims of a row, 4.7 ns a position) go over
+    // the CUs in rounds of 256, each round up to three on a CU adding to the
+    // launch, the rows form's waves run over the whole window with less company.
+    // So its line falls with the round and rises with the window.  Rows
+    // form minus decode form, us (8 / 4 heads of 256 dims; other shapes
+    // within 1 us), by workgroups and widest window:
+    //   f16        60    120    200    500    700   1000   2000
+    //    256     +2.2   +3.2   +5.1   +9.8  +13.4  +18.8
+    //    512     -0.5   -1.1   +0.5   +4.3   +7.8  +10.9  +23.4
+    //    768     -4.4   -4.5   -4.1   -1.8   +0.7   +2.8  +11.0
+    //   1024     -8.1   -8.5   -8.4   -5.9   -5.6   -5.3   -1.5
+    //   Q8_0
+    //    256     +4.0   +5.5   +9.3  +18.9  +26.0  +36.2
+    //    512     +1.6   +1.7   +4.5  +12.9  +19.6  +27.7
+    //    768     -2.6   -1.7    0.0   +6.6  +13.0  +19.6
+    //   1024     -6.5   -5.3   -4.7   +1.6   +5.6  +10.6
+    //   1280    -11.2  -11.2  -10.3   -6.5   -3.3   +0.2  +18.4
     const int64_t wgs = (int64_t)rows * n_heads * (head_dim / kSVD);
-    p.rows_form = !(wgs <= 512 || (wgs <= 1024 && p.span > 512)) &&
-                  attn_rows_v_ok(n_kv_heads, head_dim, v_fmt, capacity);
+    const int from = v_fmt == 0 ? (wgs <= 256 ? 0 : wgs <= 512 ? 150 : wgs <= 768 ? 650 : INT32_MAX)
+                                : (wgs <= 256 ? 0 : wgs <= 512 ? 40 : wgs <= 768 ? 200 : wgs <= 1024 ? 430
+                                                                    : wgs <= 1280 ? 1000 : INT32_MAX);
+    p.rows_form = p.span <= from && attn_rows_v_ok(n_kv_heads, head_dim, v_fmt, capacity);
 
     // Windows up to 256 positions: one wave a row and head, no barrier to wait
     // at (200 rows x 8 heads, window 20: 29.7 us, 27.3 with it, whole attention).
@@ -153,14 +169,16 @@ inline AttnRowsPlan attn_rows_plan(int n_past0, int rows, int n_heads, int n_kv_
     // has more than about one wave a SIMD (1024).  us at (4,2) / (4,1) / (2,1) /
     // (1,1), whole attention:
     //   f16, 256 dims: 1280 waves of (1,1) behind 2500 positions 149 / 115 / 99 / 120,
-    //     1024 behind 700 - / - / 35.5 / 34.4; 1200 of (4,1) 211 / 177 / 203 / 273,
-    //     640 38.2 / 33.3 / 32.8 / 37.5; (4,2) is level with (4,1) at 2000 waves of
-    //     its own (behind 0 / 300 / 2500 positions: 79 / 76, 105 / 104, 384 / 405);
+    //     1024 behind 700 - / - / 35.5 / 34.4; (4,1) from 800 waves of it (960 behind
+    //     700 - / 55.3 / 56.9, 640 38.2 / 33.3 / 32.8 / 37.5), later where a wave has
+    //     a whole head (8 / 8 heads of 64, 1000: 274 / 236 / 223 / 296); (4,2) is
+    //     level with (4,1) at 2000 waves of its own (behind 0 / 300 / 2500
+    //     positions: 79 / 76, 105 / 104, 384 / 405);
     //   Q8_0, where a lane's one dim is a byte load: (4,1) is never the best,
     //     (4,2) is from 400 (behind 300, 320: 42.4 / 50.8 / 42.1 / 53.0, 600: 52 / 64 /
     //     60 / 84);
-    //   Q4_0: (4,1) from 512 (640: 45.1 / 38.3 / 42.3 / 53.1, 320: 41.6 / 35.5 / 32.3
-    //     / 41.5); (4,2), a byte a lane, from 1000 where a head is two of its
+    //   Q4_0: (4,1) from 600 (640: 45.1 / 38.3 / 42.3 / 53.1, 512 with Q8_0 keys behind
+    //     2500 - / 160 / 138); (4,2), a byte a lane, from 1000 where a head is two of its
     //     slices (1200 behind 2500: 340 / 376), later where it is one (16 / 4
     //     heads of 128, 2000: 178 / 167).
     // A lane of two dims needs 128 of them, but for Q8_0.  Windows up to 160
@@ -173,7 +191,7 @@ inline AttnRowsPlan attn_rows_plan(int n_past0, int rows, int n_heads, int n_kv_
     };
     const bool ends = p.span <= 160, lanes2 = head_dim > 64 || v_fmt == 1;
     const int min42 = ends ? 1536 : v_fmt == 0 ? 2 * kSIMDs : v_fmt == 1 ? 400 : head_dim >= 256 ? 1000 : 2400;
-    const int min41 = v_fmt == 0 ? kSIMDs : kSIMDs / 2;
+    const int min41 = v_fmt != 0 ? 600 : head_dim > 64 ? 800 : 1536;
     p.pv_m = 1, p.pv_d = 1;
     if (lanes2 && waves(4, 2) >= min42) p.pv_m = 4, p.pv_d = 2;
     else if (v_fmt != 1 && !ends && waves(4, 1) >= min41) p.pv_m = 4;

@@ -86,6 +86,17 @@ def test_few_rows_take_the_decode_scores(plan):
     assert plan([attn_line(8, 8, 64, 0, 0, 4096, 200, 1000, 10)])[0]["one_row_scores"] == 1
 
 
+# (V format, workgroups of the decode form, widest window) -> the rows form measured the faster
+LINE = {(0, 256, 10): 0, (0, 512, 60): 1, (0, 512, 200): 0, (0, 768, 500): 1, (0, 768, 1000): 0, (0, 1024, 2000): 1,
+        (1, 256, 10): 0, (1, 512, 20): 1, (1, 512, 60): 0, (1, 768, 120): 1, (1, 768, 500): 0, (1, 1024, 350): 1,
+        (1, 1024, 1000): 0, (2, 1280, 700): 1, (2, 1280, 2000): 0, (2, 1536, 1000): 1}
+
+
+def test_line_between_decode_and_rows_form(plan):
+    got = plan([attn_line(8, 4, 256, vf, vf, 4096, None, span - wgs // 64, wgs // 64) for vf, wgs, span in LINE])
+    assert [p["rows_form"] for p in got] == list(LINE.values())
+
+
 # (heads, kv heads, dims, V format, window, start, batch) -> chain rows a wave x dims a lane of the weighted sum,
 # measured the fastest of the four there
 PV = {(8, 4, 256, 0, None, 2500, 40): [2, 1], (8, 4, 256, 0, None, 2500, 80): [2, 1],
