@@ -643,7 +643,99 @@ __global__ __launch_bounds__(256) void attn_rows_pv_kernel(const float *__restri
     }
 }
 
+// ---- softmax and weighted sum in one launch ---------------------------------------
+// Workgroup (head, row) where every head has its own K/V head, short windows
+// of f16 rows of 256 dims: thread d forms four weights (kept in LDS), then runs
+// dim d's chain, 32 positions in flight, the first of them loaded ahead of the
+// softmax.  Such a launch is bound by its latencies, so a second launch, or a
+// softmax for each 32 dims, costs more than the kernels above save (the line
+// and its figures: plans.h).
+__global__ __launch_bounds__(kRowsShortHD) void attn_rows_short_kernel(const float *__restrict__ scores,
+                                                                       const uint16_t *__restrict__ v_cache,
+                                                                       int n_past0, int n_heads, int capacity,
+                                                                       int wlimit, int expf_fused,
+                                                                       float *__restrict__ out)
+{
+    constexpr int HD = kRowsShortHD, B = 32;
+    __shared__ __align__(16) float p_s[kRowsShortMax];
+    __shared__ float red[HD / 64];
+    __shared__ uint64_t exp_tab[32];
+    __shared__ __align__(16) mrml_xsum::Shared4 xs;
+    const int h = blockIdx.x, z = (int)gridDim.y - 1 - (int)blockIdx.y, d = threadIdx.x;  // longest rows first
+    int window, start;
+    attn_window(nullptr, n_past0 + z, wlimit, window, start);
+    const float *sc = scores + ((size_t)z * n_heads + h) * capacity;
+    const size_t kv_dim = (size_t)n_heads * HD;
+    const uint16_t *vb = v_cache + (size_t)h * HD + d;
+    int row = (int)cache_row_of(start, capacity);  // the window's rows are consecutive modulo capacity
+    // (rows past the window are cache rows too: they are loaded, not added)
+    auto load = [&](uint16_t (&v)[B]) {
+#pragma unroll
+        for (int k = 0; k < B; ++k) {
+            v[k] = vb[(size_t)row * kv_dim];
+            row = row + 1 == capacity ? 0 : row + 1;
+        }
+    };
+    uint16_t va[B], vn[B];
+    load(va);  // in flight during the softmax
+    if (d < 32) exp_tab[d] = mrml_libm::kExpfT.t[d];
+    float sv[4], mx = -INFINITY;  // the max is exact in any order
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        sv[i] = 4 * d + i < window ? sc[4 * d + i] : -INFINITY;
+        mx = fmaxf(mx, sv[i]);
+    }
+    mx = max32(mx);
+    mx = fmaxf(mx, __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mx), 32)));
+    if ((d & 63) == 0) red[d >> 6] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    float e[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        e[i] = 4 * d + i < window ? mrml_libm::expf_t(sv[i] - mx, expf_fused != 0, exp_tab) : 0.0f;
+    const float sum = mrml_xsum::block_seq_sum_nonneg4(make_float4(e[0], e[1], e[2], e[3]), window, xs);
+    const float inv = sum > 0.0f ? 1.0f / sum : 1.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (4 * d + i < window) p_s[4 * d + i] = sum > 0.0f ? e[i] * inv : e[i];
+    __syncthreads();
+
+    float acc = 0.0f;
+    auto add = [&](const uint16_t (&v)[B], int t0) {
+        if (t0 + B <= window) {
+#pragma unroll
+            for (int i = 0; i < B; i += 4) {
+                const float4 p4 = *reinterpret_cast<const float4 *>(p_s + t0 + i);
+                acc = acc + p4.x * f16_bits_to_f32(v[i]);
+                acc = acc + p4.y * f16_bits_to_f32(v[i + 1]);
+                acc = acc + p4.z * f16_bits_to_f32(v[i + 2]);
+                acc = acc + p4.w * f16_bits_to_f32(v[i + 3]);
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < B; ++k)
+                if (t0 + k < window) acc = acc + p_s[t0 + k] * f16_bits_to_f32(v[k]);
+        }
+    };
+    for (int t0 = 0; t0 < window; t0 += 2 * B) {
+        if (t0 + B < window) load(vn);  // in flight while va is added
+        add(va, t0);
+        if (t0 + 2 * B < window) load(va);
+        if (t0 + B < window) add(vn, t0 + B);
+    }
+    out[((size_t)z * n_heads + h) * HD + d] = acc;
+}
+
 }  // namespace
+
+int launch_attn_rows_short(mrml_hip_ctx *ctx, const float *scores, const void *v_cache, float *out, int n_past0,
+                           int rows, int n_heads, int capacity, int wlimit)
+{
+    hipLaunchKernelGGL(attn_rows_short_kernel, dim3(n_heads, rows), dim3(kRowsShortHD), 0, ctx->stream, scores,
+                       (const uint16_t *)v_cache, n_past0, n_heads, capacity, wlimit, (int)host_expf_fused(), out);
+    return check_launch(ctx, "attn_rows_short_kernel");
+}
 
 int launch_attn_rows_scores(mrml_hip_ctx *ctx, const AttnRowsPlan &plan, const float *q, int q_stride,
                             const void *k_cache, int n_past0, int rows, int n_heads, int n_kv_heads, int head_dim,

@@ -1699,6 +1699,8 @@ int launch_attn_rows(mrml_hip_ctx *ctx, const float *q, int q_stride, const void
                        : launch_attn_rows_scores(ctx, plan, q, q_stride, k_cache, n_past0, rows, n_heads, n_kv_heads,
                                                  head_dim, k_fmt, scale, capacity, wlimit, scores);
     if (rc) return rc;
+    if (plan.short_form)
+        return launch_attn_rows_short(ctx, scores, v_cache, out, n_past0, rows, n_heads, capacity, wlimit);
     if (!plan.rows_form)
         return launch_softmax_v(ctx, scores, v_cache, out, nullptr, nullptr, n_past0, n_heads, n_kv_heads, capacity,
                                 wlimit, rows, head_dim, v_fmt);

@@ -219,6 +219,8 @@ int launch_attn_rows(mrml_hip_ctx *ctx, const float *q, int q_stride, const void
 int launch_attn_rows_scores(mrml_hip_ctx *ctx, const AttnRowsPlan &plan, const float *q, int q_stride,
                             const void *k_cache, int n_past0, int rows, int n_heads, int n_kv_heads, int head_dim,
                             int k_fmt, float scale, int capacity, int wlimit, float *scores);
+int launch_attn_rows_short(mrml_hip_ctx *ctx, const float *scores, const void *v_cache, float *out, int n_past0,
+                           int rows, int n_heads, int capacity, int wlimit);
 int launch_attn_rows_softmax_v(mrml_hip_ctx *ctx, const AttnRowsPlan &plan, float *scores, const void *v_cache,
                                float *out, int n_past0, int rows, int n_heads, int n_kv_heads, int head_dim, int v_fmt,
                                int capacity, int wlimit);

@@ -39,6 +39,8 @@ __host__ __device__
 #endif
 constexpr int rows_k_stride(int head_dim) { return head_dim * 2 + 16; }  // bytes of a staged f16 K row
 
+constexpr int kRowsShortHD = 256, kRowsShortMax = 112;  // dims and positions of the short form
+
 struct AttnRowsPlan {
     int span;             // the widest window
     int t_lo;             // the first row's window start
@@ -47,6 +49,7 @@ struct AttnRowsPlan {
     int score_reps;       // passes over a staged tile
     int tiles;            // score tiles dispatched a row block
     bool all_tiles;       // those are all from t_lo to the last row's position
+    bool short_form;      // softmax and weighted sum in one launch (attn_rows_short_kernel), else
     bool rows_form;       // softmax and weighted sum as attn_rows.hip has them, else the decode form
     int softmax_threads;
     int pv_m, pv_d;       // weighted sum: chain rows a wave, dims a lane
@@ -153,6 +156,18 @@ inline AttnRowsPlan attn_rows_plan(int n_past0, int rows, int n_heads, int n_kv_
                                 : (wgs <= 256 ? 0 : wgs <= 512 ? 40 : wgs <= 768 ? 200 : wgs <= 1024 ? 430
                                                                     : wgs <= 1280 ? 1000 : INT32_MAX);
     p.rows_form = p.span <= from && attn_rows_v_ok(n_kv_heads, head_dim, v_fmt, capacity);
+
+    // One launch for both, us against the choice above (8 / 8 heads, whole
+    // attention): against the decode form in its first round of workgroups, 1 row at
+    // 0 10.9 / 11.5, at 60 13.2 / 11.6; after it, 16 rows at 60 14.8 / 15.6, at 100
+    // 16.0 / 15.8; 64 rows from 0 14.2 / 15.2, 50 at 60 18.2 / 17.4; a window of 60,
+    // 64 rows 15.4 / 16.4, 130 22.1 / 22.6 (16 / 16 heads, 50: 19.4 / 18.9); of
+    // 20, 200 rows 22.4 / 25.7.
+    const int64_t heads = (int64_t)rows * n_heads;
+    p.short_form = group == 1 && head_dim == kRowsShortHD && v_fmt == 0 &&
+                   (wgs <= kCUs ? p.span <= 16
+                                : p.span <= 32 || (p.span <= 64 && heads <= 3 * kCUs) ||
+                                      (p.span <= kRowsShortMax && heads <= kCUs));
 
     // Windows up to 256 positions: one wave a row and head, no barrier to wait
     // at (200 rows x 8 heads, window 20: 29.7 us, 27.3 with it, whole attention).

@@ -21,8 +21,8 @@ int main()
             const AttnRowsPlan p = attn_rows_plan(a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8]);
             const int nchains = a[1] * (a[2] / a[3]);
             std::printf("{\"span\": %d, \"tiles\": %d, \"score_m\": %d, \"score_reps\": %d, \"score_blocks\": %d, "
-                        "\"one_row_scores\": %d, \"rows_form\": %d, \"softmax_threads\": %d, \"pv\": [%d, %d], \"long\": %d}\n",
-                        p.span, p.tiles, p.score_m, p.score_reps, p.score_blocks(nchains), p.one_row_scores, p.rows_form,
+                        "\"one_row_scores\": %d, \"short_form\": %d, \"rows_form\": %d, \"softmax_threads\": %d, \"pv\": [%d, %d], \"long\": %d}\n",
+                        p.span, p.tiles, p.score_m, p.score_reps, p.score_blocks(nchains), p.one_row_scores, p.short_form, p.rows_form,
                         p.softmax_threads, p.pv_m, p.pv_d, sv_long(p.span));
         } else if (!std::strcmp(op, "gemm")) {
             int rows, batch;

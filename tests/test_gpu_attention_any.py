@@ -244,6 +244,12 @@ MANY_ROWS = [
     (8, 8, 64, 0, 0, 300, 90, 280, 21),        # scores a workgroup a row: any head size, the ring's end inside
     (9, 3, 32, 0, 0, 128, None, 0, 70),
     (6, 2, 256, 0, 0, 200, 70, 190, 40),       # and 256 dims, group of 3
+    # softmax and sum in one launch: windows of 1 to 60 positions, sliding ones, the ring's end inside
+    (8, 8, 256, 0, 0, 512, None, 0, 60),
+    (16, 16, 256, 0, 0, 40, 32, 70, 20),
+    (8, 8, 256, 0, 0, 512, 1, 40, 12),
+    (4, 4, 256, 0, 0, 110, None, 180, 64),
+    (2, 2, 256, 0, 0, 64, 63, 10, 100),
     # the long softmax with several rows, at every value format; the second and third across whole chunks
     (4, 2, 64, 0, 0, 16384, None, 11000, 3),
     (4, 2, 64, 1, 1, 16384, None, 16380, 4),

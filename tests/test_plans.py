@@ -97,6 +97,19 @@ def test_line_between_decode_and_rows_form(plan):
     assert [p["rows_form"] for p in got] == list(LINE.values())
 
 
+# (heads = kv heads, window, start, batch) -> whether softmax and sum in one launch measured the faster
+SHORT = {(8, None, 0, 1): 1, (8, None, 60, 1): 0, (8, None, 0, 64): 1, (8, None, 60, 16): 1, (8, None, 60, 50): 0,
+         (8, None, 200, 9): 0, (8, 20, 1000, 200): 1, (8, 60, 1000, 64): 1, (16, 60, 1000, 100): 0}
+
+
+def test_short_windows_of_single_heads_in_one_launch(plan):
+    got = plan([attn_line(h, h, 256, 0, 0, 4096, sw, start, batch) for h, sw, start, batch in SHORT])
+    assert [p["short_form"] for p in got] == list(SHORT.values())
+    others = [attn_line(8, 4, 256, 0, 0, 4096, 20, 1000, 64), attn_line(8, 8, 128, 0, 0, 4096, 20, 1000, 64),
+              attn_line(8, 8, 256, 0, 1, 4096, 20, 1000, 64)]
+    assert [p["short_form"] for p in plan(others)] == [0, 0, 0]
+
+
 # (heads, kv heads, dims, V format, window, start, batch) -> chain rows a wave x dims a lane of the weighted sum,
 # measured the fastest of the four there
 PV = {(8, 4, 256, 0, None, 2500, 40): [2, 1], (8, 4, 256, 0, None, 2500, 80): [2, 1],
@@ -123,7 +136,9 @@ def test_prefill_cases_reach_every_form(plan):
             scores.add("tuned" if hd == 256 else "any")
         else:
             scores.add((kf, p["score_m"], min(p["score_reps"], 2)))
-        if p["rows_form"]:
+        if p["short_form"]:
+            weighted.add("short")
+        elif p["rows_form"]:
             chunks = p["span"] > 4 * p["softmax_threads"]
             softmax.add((p["softmax_threads"], chunks))
             weighted.add((vf, *p["pv"]))
@@ -134,4 +149,4 @@ def test_prefill_cases_reach_every_form(plan):
     assert softmax >= {(64, False), (256, False), (256, True), (512, False), (1024, False), (1024, True)}
     forms = [(4, 2), (4, 1), (2, 1), (1, 1)]
     assert weighted >= {(vf, *f) for vf in range(3) for f in forms if (vf, f) != (1, (4, 1))}  # (not built)
-    assert weighted >= {(vf, f) for vf in range(3) for f in ("decode", "long")}
+    assert weighted >= {(vf, f) for vf in range(3) for f in ("decode", "long")} | {"short"}
