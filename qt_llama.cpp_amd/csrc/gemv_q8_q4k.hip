@@ -3,6 +3,8 @@
 // kernels (one 16-lane DPP row per matrix row, 4 rows per wave); this file
 // is compiled with -ffp-contract=off.
 
+#include <type_traits>
+
 #include "device.h"
 #include "internal.h"
 #include "libm_f32.h"
@@ -777,27 +779,32 @@ __global__ __launch_bounds__(kSelectThreads) void vocab_select_kernel(
         return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
     };
     int token = n ? __builtin_amdgcn_readlane(id, 0) : 506;
-    if (n > 0 && temperature > 0.0f) {
+    if (n > 1 && temperature > 0.0f) {  // (a single candidate is drawn whatever its weight)
         // the CPU path's state.pos: the position after the token just processed
         const unsigned long long pos = state ? (unsigned long long)state[1] + 1ull : pos_arg;
         const float s0 = lane_f32(score, 0);
         const float temp = temperature > 0.1f ? temperature : 0.1f;
         const float prob = t < n ? mrml_libm::expf((score - s0) / temp, expf_fused != 0) : 0.0f;
-        float sum_exp = 0.0f;
+        // over the first N lanes' candidates (+ 0 past them)
+        auto draw = [&](auto lanes) {
+            constexpr int N = decltype(lanes)::value;
+            float sum_exp = 0.0f;
 #pragma unroll
-        for (int i = 0; i < kTopKMax; ++i) sum_exp += lane_f32(prob, i);  // (+ 0 past the candidates)
-        if (sum_exp > 0.0f) {
+            for (int i = 0; i < N; ++i) sum_exp += lane_f32(prob, i);
+            if (!(sum_exp > 0.0f)) return;
             const float quot = prob / sum_exp;
             const float rng = (float)((pos * 6364136223846793005ull + 1ull) >> 33) / (float)0xffffffffu;
             float acc = 0.0f, mine = 0.0f;  // mine: the sum up to this lane's candidate
 #pragma unroll
-            for (int i = 0; i < kTopKMax; ++i) {
+            for (int i = 0; i < N; ++i) {
                 acc += lane_f32(quot, i);
                 mine = t == i ? acc : mine;
             }
             const uint64_t hit = __ballot(t < n && rng <= mine);
             if (hit) token = __builtin_amdgcn_readlane(id, __builtin_ctzll(hit));
-        }
+        };
+        if (k <= 8) draw(std::integral_constant<int, 8>{});
+        else draw(std::integral_constant<int, kTopKMax>{});
     }
     if (t != 0) return;
     if (out_token) *out_token = token;

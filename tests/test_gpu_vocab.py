@@ -106,6 +106,25 @@ def test_vocab_select_forms(backend, dev, orc, vocab, shape):
                          f"vocab={vocab} {shape} k={k} scoring={scoring}")
 
 
+# The draw on both sides of its two widths (8 and 64 lanes), at positions that
+# spread the random number, over candidates from all of k down to one (the
+# weights so unequal, or the candidates so few, that the first takes all).
+@pytest.mark.parametrize("k", [1, 2, 7, 8, 9, 63])
+def test_vocab_draw_widths(backend, dev, orc, k):
+    vocab = 5000
+    rng = np.random.default_rng(k)
+    lg = (rng.standard_normal(vocab) * 3.0).astype(np.float32)
+    recent = rng.integers(0, vocab, 32).astype(np.int32)
+    for keep in (vocab, 8, 1):
+        valid = np.zeros(vocab, np.uint8)
+        valid[rng.permutation(np.arange(200, vocab))[:keep]] = 1
+        bufs = [backend.HipBuffer.from_host(dev, a) for a in (lg, valid, recent)]
+        for temp in (0.05, 1.0, 25.0):
+            for pos in range(3, 2 ** 20, 2 ** 17):
+                check_select(backend, dev, orc, *bufs, lg, valid, recent, 0, 9, temp, pos, k,
+                             f"k={k} keep={keep} t={temp} pos={pos}")
+
+
 def partition_bounds(vocab: int, parts: int, p: int):
     return vocab * p // parts, vocab * (p + 1) // parts
 
