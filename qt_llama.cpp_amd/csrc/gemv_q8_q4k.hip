@@ -353,6 +353,10 @@ template <int P, typename T, typename F>
 __device__ __forceinline__ int count_if(const T *vals, int n, F pass)
 {
     int c = 0;
+    if constexpr (P == 1) {  // (with n constant, reads of 16 bytes and no tail to test)
+        for (int u = 0; u < n; ++u) c += pass(vals[u]) ? 1 : 0;
+        return c;
+    }
     for (int u0 = (int)threadIdx.x % P; u0 < n; u0 += 8 * P) {
         T x[8];
 #pragma unroll
