@@ -172,14 +172,17 @@ def test_gemm_q4_0_split_tiles_bit_exact(backend, dev, orc, synth, rows, cols, b
 # Few tokens (16 rows x 16 tokens a workgroup, rounds of 32 or 16 blocks): one
 # block, partial and whole last rounds of an odd and even number, ragged row
 # and token tiles, both producer counts (448 workgroups and more take the
-# smaller), and the two sides of the line to the tile kernel (2304
-# workgroups), the tile kernel's with a K tail.
-@pytest.mark.parametrize("rows,cols,batch", [
+# smaller), and the two sides of the line to the tile kernel, the tile kernel's
+# with a K tail.  (test_plans.py says which side each is on.)
+FEW_CASES = [
     (17, 32, 1), (16, 96, 2), (40, 31 * 32, 15), (33, 32 * 32, 16), (5, 33 * 32, 17), (47, 64 * 32, 31),
     (16, 65 * 32, 33), (31, 512 * 32, 3),
     (7168, 15 * 32, 5), (7153, 16 * 32, 16), (3600, 17 * 32, 19), (7185, 33 * 32, 2),
     (9216, 13 * 32, 64), (9216, 13 * 32, 65),
-])
+]
+
+
+@pytest.mark.parametrize("rows,cols,batch", FEW_CASES)
 def test_gemm_q4_0_few_tokens_bit_exact(backend, dev, orc, synth, rows, cols, batch):
     rng = synth.rng_for(5180 + rows + cols + batch)
     w = synth.q4_0_matrix(rng, rows, cols)
@@ -198,6 +201,62 @@ def test_gemm_q4_0_few_tokens_bit_exact(backend, dev, orc, synth, rows, cols, ba
     u = oracle_gemm(orc, w2, x, rows, cols, range(batch))
     assert_bit_exact(ab.numpy().reshape(batch, rows), np.stack([orc.geglu(ref[m], u[m]) for m in range(batch)]),
                      "geglu")
+
+
+# The tile kernel, past the few-token line: K of less than one 8-block chunk,
+# of whole chunks and every tail after them, with an odd number of rows (scalar
+# stores, a partial last row tile) in FULL waves (5101 rows) and in the HALF
+# waves that end a launch of just over one a SIMD (9217 rows), partial token
+# groups; rows of whole tiles (16-byte stores).
+TILE_CASES = [(5101, 32 * nb, 113 + 2 * (nb % 8)) for nb in (1, 2, 3, 4, 5, 6, 7, 9, 10, 11, 12, 13, 14, 15, 16)] + [
+    (9217, 32, 65), (9217, 3 * 32, 70), (9217, 7 * 32, 128), (9217, 12 * 32, 97), (9217, 14 * 32, 66),
+    (5120, 5 * 32, 128), (9216, 9 * 32, 100), (4608, 15 * 32, 128)]
+
+
+@pytest.mark.parametrize("rows,cols,batch", TILE_CASES)
+def test_gemm_q4_0_tiles_bit_exact(backend, dev, orc, synth, rows, cols, batch):
+    rng = synth.rng_for(5185 + rows + cols + batch)
+    w = synth.q4_0_matrix(rng, rows, cols)
+    x = (rng.standard_normal((batch, cols)) * 10.0 ** rng.uniform(-3, 3, (batch, 1))).astype(np.float32)
+    x[batch - 1, :32] = 0.0
+    got = run_gemm(backend, dev, w, x, rows, cols, batch)
+    assert_bit_exact(got, oracle_gemm(orc, w, x, rows, cols, range(batch)), f"gemm {rows}x{cols} M={batch}")
+
+
+def test_gemm_q4_0_tiles_integer_accumulators(backend, dev):
+    """test_gemm_q4_0_integer_accumulators on the tile kernel."""
+    rows, cols, batch = 9216, 32, 200
+    rng = np.random.default_rng(78)
+    nib = rng.integers(0, 16, (rows, 32))
+    nib[0], nib[1], nib[rows - 1] = 0, 15, 0
+    q = rng.integers(-127, 128, (batch, 32))
+    q[:, 0] = 127
+    q[1, 1:] = -127
+    w = np.zeros((rows, 18), np.uint8)
+    w[:, 1] = 0x3C  # f16 1.0
+    w[:, 2:] = (nib[:, :16] | (nib[:, 16:] << 4)).astype(np.uint8)
+    got = run_gemm(backend, dev, w.reshape(-1), q.astype(np.float32), rows, cols, batch)
+    isum = q.astype(np.int64) @ (nib - 8).T.astype(np.int64)
+    assert np.array_equal(got, isum.astype(np.float32)), "integer block dots differ"
+
+
+@pytest.mark.parametrize("q_rows,kv_rows", [(5101, 1501), (5120, 1504)])
+def test_gemm_q4_0_qkv_tiles(backend, dev, orc, synth, q_rows, kv_rows):
+    """The stacked product past the few-token line: one launch over whole row
+    tiles, and row counts that are none (q in tiles, k and v by the few-token
+    kernel, each at its column offset of an odd row stride)."""
+    cols, batch = 7 * 32, 128
+    rng = synth.rng_for(5186 + q_rows)
+    ws = [synth.q4_0_matrix(rng, r, cols) for r in (q_rows, kv_rows, kv_rows)]
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    bufs = [backend.HipBuffer.from_gguf(dev, w, backend.Q4_0, r, cols) for w, r in zip(ws, (q_rows, kv_rows, kv_rows))]
+    xb = backend.HipBuffer.from_host(dev, x.reshape(-1))
+    yb = backend.HipBuffer.alloc(dev, batch * (q_rows + 2 * kv_rows))
+    dev.gemm_q4_0_qkv(*bufs, xb, yb, q_rows, kv_rows, cols, batch)
+    dev.sync()
+    ref = np.concatenate([oracle_gemm(orc, w, x, r, cols, range(batch))
+                          for w, r in zip(ws, (q_rows, kv_rows, kv_rows))], axis=1)
+    assert_bit_exact(yb.numpy().reshape(batch, -1), ref, "qkv")
 
 
 def test_gemm_q4_0_qkv_geglu_any_rows(backend, dev, orc, synth):
