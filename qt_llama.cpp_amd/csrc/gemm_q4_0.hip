@@ -731,7 +731,7 @@ static int launch_gemm_mats(mrml_hip_ctx *ctx, const GemmMats &mats, const void 
     if (ldy < rows || ((uintptr_t)y & 3) != 0)
         return fail(ctx, MRML_HIP_E_INVALID, "gemm_q4_0: output stride %d below rows %d, or y not 4-byte aligned",
                     ldy, rows);
-    if (!relaxed && gemm_few(rows, batch)) return launch_gemm_few(ctx, false, mats, gpack, y, rows, nb, batch, ldy);
+    if (!relaxed && gemm_few(rows, nb, batch, false)) return launch_gemm_few(ctx, false, mats, gpack, y, rows, nb, batch, ldy);
     const int vec = (ldy % 4 == 0 && ((uintptr_t)y & 15) == 0) ? 1 : 0;  // float4 stores reach every output row
     const int rt = (rows + 31) / 32, gq = (ng + kGemmWaves - 1) / kGemmWaves;
     const int rt_full = gemm_full_tiles(rows, batch);
@@ -760,7 +760,7 @@ int launch_gemm_q4_0(mrml_hip_ctx *ctx, const void *w, const void *gpack, float 
 int launch_gemm_q4_0_geglu(mrml_hip_ctx *ctx, const void *wg, const void *wu, const void *gpack, float *act, float *gu,
                            int32_t rows, int32_t cols, int32_t batch)
 {
-    if (gemm_few(rows, batch)) {
+    if (gemm_few_glu(rows, batch)) {
         GemmMats mats{};
         mats.w[0] = (const uint8_t *)wg;
         mats.w[1] = (const uint8_t *)wu;

@@ -630,16 +630,16 @@ int prefill_buffers(mrml_hip_ctx *ctx, mrml_hip_gemma2 *m)
 }
 
 // FAST numerics take the one-FMA GEMM fold where it is the faster one.
-inline bool relaxed_gemm(const mrml_hip_gemma2_config &c, int rows, int n)
+inline bool relaxed_gemm(const mrml_hip_gemma2_config &c, int rows, int cols, int n)
 {
-    return c.numerics == MRML_HIP_NUMERICS_FAST && !gemm_few(rows, n);
+    return c.numerics == MRML_HIP_NUMERICS_FAST && !gemm_few(rows, cols / 32, n, true);
 }
 
 // Q8_0 of n rows of `cols` f32 values as a GEMM pack, then y = W * x for every row.
 int gemm_rows(mrml_hip_ctx *ctx, mrml_hip_gemma2 *m, const void *w, const float *x, float *y, int rows, int cols, int n)
 {
     if (int rc = launch_gemm_pack_quantize(ctx, x, m->pf_gpack, cols, n)) return rc;
-    return launch_gemm_q4_0(ctx, w, m->pf_gpack, y, rows, cols, n, 0, relaxed_gemm(m->cfg, rows, n));
+    return launch_gemm_q4_0(ctx, w, m->pf_gpack, y, rows, cols, n, 0, relaxed_gemm(m->cfg, rows, cols, n));
 }
 
 }  // namespace
@@ -691,7 +691,7 @@ int mrml_hip_gemma2_prefill(mrml_hip_ctx *ctx, mrml_hip_gemma2 *m, const int32_t
                 const void *qkv_w[3] = {L.wq, L.wk, L.wv};
                 const int32_t qkv_rows[3] = {qd, kvd, kvd};
                 STEP(launch_gemm_q4_0_stacked(ctx, qkv_w, qkv_rows, 3, m->pf_gpack, m->pf_qkv, c.dim, n, qkvd,
-                                              relaxed_gemm(c, qkvd, n)));
+                                              relaxed_gemm(c, qkvd, c.dim, n)));
             }
             if ((int64_t)p0 + n > c.ctx_len) {
                 // The chunk wraps the ring: a later token's K/V row replaces
@@ -725,14 +725,14 @@ int mrml_hip_gemma2_prefill(mrml_hip_ctx *ctx, mrml_hip_gemma2 *m, const int32_t
             const void *gu_w[2] = {L.w_gate, L.w_up};
             const int32_t gu_rows[2] = {c.ffn_dim, c.ffn_dim};
             STEP(launch_gemm_q4_0_stacked(ctx, gu_w, gu_rows, 2, m->pf_gpack, m->pf_gu, c.dim, n, 0,
-                                          relaxed_gemm(c, 2 * c.ffn_dim, n)));
+                                          relaxed_gemm(c, 2 * c.ffn_dim, c.dim, n)));
             // act = gelu_tanh(g) * u per element (the GeGLU epilogue of the
             // matvec kernels, so each act value has the token step's bits),
             // quantized into the down projection's pack as it is formed
             STEP(launch_gemm_pack_geglu(ctx, m->pf_gu, m->pf_gu + c.ffn_dim, 2 * c.ffn_dim, m->pf_gpack, c.ffn_dim,
                                         n));
             STEP(launch_gemm_q4_0(ctx, L.w_down, m->pf_gpack, m->pf_f, c.dim, c.ffn_dim, n, 0,
-                                  relaxed_gemm(c, c.dim, n)));
+                                  relaxed_gemm(c, c.dim, c.ffn_dim, n)));
             STEP(launch_residual_rms_norm(ctx, m->pf_f, L.post_ffw_norm, h, h, next_norm, c.eps, xn, nullptr, c.dim,
                                           n, fast, l + 1 < c.n_layers ? m->pf_gpack : nullptr));
         }

@@ -223,16 +223,31 @@ inline int64_t few_workgroups(int32_t rows, int32_t batch)
     return (int64_t)((rows + kFewRows - 1) / kFewRows) * ((batch + kFewTokens - 1) / kFewTokens);
 }
 
-// Whether an exact product runs as gemm_q4_0_few_kernel (a relaxed one never
-// does: the tile kernel's one-FMA fold is slower there than the few-token
-// kernel's exact one).  A workgroup costs about 8.5e-5 us a block there once
-// the chip is full; the tile kernel takes 0.2 us a block for anything up to
-// one wave a SIMD (a lone wave's step), so the line is at 0.2 / 8.5e-5
-// workgroups.  Measured on both sides of it:
-// 9216 x 2304 at 64 tokens (2304 workgroups) 17.6 against 19.7 us, at 80
-// (2880) 21.4 against 20.0; 4096 x 2304 at 128 (2048) 15.5 against 18.1;
-// 2304 x 9216 at 128 (1152) 28.4 against 58.7.
-inline bool gemm_few(int32_t rows, int32_t batch) { return few_workgroups(rows, batch) <= 2304; }
+// Whether a product of nb-block rows runs as gemm_q4_0_few_kernel, whose fold
+// is exact, or in tiles (relaxed: with their one-FMA fold; the entry that asks
+// for that fold always gets it).  A few-token workgroup costs about 1 ns and
+// 8.5e-5 us a block once the chip is full; the tile kernel takes 0.2 us a block
+// for anything up to one wave a SIMD (a lone wave's step), so the line rises
+// with K.  us, few / tiles / relaxed tiles, at 2048, 2304 and 2560 workgroups
+// (4096, 4608, 5120 rows, 128 tokens):
+//   K  512   13.3 / 13.6 / 13.0   14.1 / 13.5 / 13.0   14.7 / 13.6 / 13.2
+//   K 2304   22.6 / 24.2 / 22.4   24.1 / 24.7 / 22.6   25.7 / 24.6 / 22.7
+//   K 4096   29.2 / 35.3 / 31.6   31.2 / 36.0 / 32.1   33.5 / 35.8 / 32.3
+//   K 9216   51.9 / 66.5 / 59.4   57.0 / 68.0 / 60.1   61.5 / 67.2 / 59.1
+// Few tokens leave the tiles' workgroups of four token groups with less than
+// four waves' work: 18432 rows x 32 tokens (2304) at K 2304 24.0 / 35.4 / 33.2.
+inline bool gemm_few(int32_t rows, int nb, int32_t batch, bool relaxed)
+{
+    const int64_t w = few_workgroups(rows, batch), groups = (batch + 31) / 32;
+    if (w <= 2048 || w > 2304) return w <= 2048;
+    const int64_t waves = (int64_t)((rows + 31) / 32) * ((groups + kGemmWaves - 1) / kGemmWaves) * kGemmWaves;
+    return waves > kSIMDs || nb >= (relaxed ? 112 : 64);
+}
+
+// And gate, up and activation together: the tiles pay twice and an
+// elementwise pass (9216 x 2304 at 64 tokens, 2304 workgroups, 38.6 / 48.5 us; 4608 x
+// 512 at 128 19.5 / 24.6).
+inline bool gemm_few_glu(int32_t rows, int32_t batch) { return few_workgroups(rows, batch) <= 2304; }
 
 // Producers of a few-token workgroup: 8 while the workgroups leave CUs their
 // LDS (two of them a CU), else 4 (up to four a CU).  2304 x 9216 at 16 tokens

@@ -1,7 +1,7 @@
 // Prints what the dispatch rules (csrc/plans.h) say of the calls on stdin,
 // one JSON object a line:
 //   attn n_past0 rows n_heads n_kv_heads head_dim k_fmt v_fmt capacity wlimit
-//   gemm rows batch
+//   gemm rows cols batch
 //   span positions
 #include <cstdio>
 #include <cstring>
@@ -25,10 +25,13 @@ int main()
                         p.span, p.tiles, p.score_m, p.score_reps, p.score_blocks(nchains), p.one_row_scores, p.short_form, p.rows_form,
                         p.softmax_threads, p.pv_m, p.pv_d, sv_long(p.span));
         } else if (!std::strcmp(op, "gemm")) {
-            int rows, batch;
-            if (std::scanf("%d %d", &rows, &batch) != 2) return 1;
-            std::printf("{\"few\": %d, \"producers\": %d, \"full_tiles\": %d, \"tiles\": %d}\n", gemm_few(rows, batch),
-                        gemm_few_producers(false, rows, batch), gemm_full_tiles(rows, batch), (rows + 31) / 32);
+            int rows, cols, batch;
+            if (std::scanf("%d %d %d", &rows, &cols, &batch) != 3) return 1;
+            std::printf("{\"few\": %d, \"few_fast\": %d, \"few_glu\": %d, \"producers\": %d, \"full_tiles\": %d, "
+                        "\"tiles\": %d}\n",
+                        gemm_few(rows, cols / 32, batch, false), gemm_few(rows, cols / 32, batch, true),
+                        gemm_few_glu(rows, batch), gemm_few_producers(false, rows, batch),
+                        gemm_full_tiles(rows, batch), (rows + 31) / 32);
         } else if (!std::strcmp(op, "span")) {
             int span;
             if (std::scanf("%d", &span) != 1) return 1;

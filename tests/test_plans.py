@@ -14,6 +14,8 @@ from pathlib import Path
 import pytest
 
 import test_gpu_attention_any as attention_any
+import test_gpu_decode as decode
+import test_gpu_gemm as gemm
 import test_gpu_prefill_ops as prefill_ops
 
 NATIVE = Path(__file__).resolve().parent / "native"
@@ -150,3 +152,38 @@ def test_prefill_cases_reach_every_form(plan):
     forms = [(4, 2), (4, 1), (2, 1), (1, 1)]
     assert weighted >= {(vf, *f) for vf in range(3) for f in forms if (vf, f) != (1, (4, 1))}  # (not built)
     assert weighted >= {(vf, f) for vf in range(3) for f in ("decode", "long")} | {"short"}
+
+
+def gemm_plans(plan, cases):
+    return plan([f"gemm {rows} {cols} {batch}" for rows, cols, batch in cases])
+
+
+def test_gemm_cases_are_on_their_side_of_the_line(plan):
+    few = [p["few"] for p in gemm_plans(plan, gemm.FEW_CASES)]
+    assert few == [1] * (len(few) - 1) + [0]
+    cases = gemm.TILE_CASES
+    plans = gemm_plans(plan, cases)
+    assert not any(p["few"] for p in plans)
+    full = [(c, p) for c, p in zip(cases, plans) if p["full_tiles"] == p["tiles"]]
+    half = [(c, p) for c, p in zip(cases, plans) if p["full_tiles"] < p["tiles"]]
+    assert {c[1] // 32 % 8 for c, _ in full if c[1] // 32 > 8} == set(range(8))  # every tail after a whole chunk
+    assert {c[1] // 32 for c, _ in full if c[1] // 32 < 8} == set(range(1, 8))   # and before any
+    for kind in (full, half):
+        assert any(c[0] % 32 and c[0] % 4 for c, _ in kind) and any(c[0] % 4 == 0 for c, _ in kind)
+
+
+# (rows, cols, batch) -> few-token kernel in EXACT, in FAST, measured as the faster one
+GEMM_LINE = {(4608, 512, 128): (0, 0), (18432, 512, 32): (1, 1), (4096, 512, 128): (1, 1), (4608, 2304, 128): (1, 0),
+             (2304, 2304, 256): (1, 0), (18432, 2304, 32): (1, 1), (5120, 2304, 128): (0, 0), (4608, 4096, 128): (1, 1),
+             (4608, 9216, 128): (1, 1), (9216, 2304, 80): (0, 0)}
+
+
+def test_few_token_line(plan):
+    got = [(p["few"], p["few_fast"]) for p in gemm_plans(plan, GEMM_LINE)]
+    assert got == list(GEMM_LINE.values())
+
+
+def test_fast_prefill_test_has_both_folds(plan):
+    layer = decode.FAST_LAYER.values()
+    got = gemm_plans(plan, [(rows, cols, 150) for rows, cols, _ in layer])
+    assert [not p["few_fast"] for p in got] == [relaxed for _, _, relaxed in layer]
