@@ -60,10 +60,14 @@ CASES = [
     (8, 4, 256, 1, 0, 768, None, [767]),
     (8, 4, 256, 0, 2, 768, None, [767]),
     (32, 2, 256, 0, 0, 256, None, [0, 255]),
-    # odd head sizes that are multiples of 32, the long softmax form (capacity past 6144)
+    # odd head sizes that are multiples of 32, softmax in register chunks, and
+    # the long form (windows past 10240) at every value format
     (6, 3, 96, 1, 1, 128, None, [0, 127]),
     (2, 1, 32, 2, 0, 64, None, [0, 63]),
     (4, 2, 160, 0, 1, 8192, None, [6000, 8191]),
+    (4, 2, 96, 2, 2, 16384, None, [10239, 10240, 16382]),
+    (4, 2, 64, 0, 1, 16384, None, [10240, 16383]),
+    (4, 2, 64, 1, 0, 16384, 16381, [17000]),
 ]
 
 

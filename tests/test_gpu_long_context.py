@@ -1,10 +1,12 @@
 """GPU parity of attention and the token step at long KV capacities (C ABI).
 
-Capacities past 6144 positions take the long forms of the attention kernels:
-the exact softmax sums the window's exps in chunks of 8191 staged in LDS,
-each chunk's exact sequential sum started from the running sum, and forms
-the weights again from the global scores; the split-K combine walks more
-tiles than its LDS arrays hold.  Bar: bit-identical to the CPU oracle
+Launches whose widest window is past 10240 positions (the whole capacity, when
+the position is on the device) take the long form of the exact softmax: it sums
+the window's exps in chunks of 8191 staged in LDS, each chunk's exact
+sequential sum started from the running sum, and forms the weights again from
+the global scores; up to there the weights stay in LDS and the sum runs in
+register chunks.  Past 6144 positions the split-K combine walks more tiles than
+its LDS arrays hold.  Bar: bit-identical to the CPU oracle
 (model.rs:1457-1590, ops.rs:133-158) for the exact path at every window up
 to 131072 positions (test_gpu_attention_any.py takes a 262144-position
 window; the ops take capacities up to 2^20); within 1e-5 relative to
@@ -33,7 +35,7 @@ def window_rows(n_past: int, cap: int) -> np.ndarray:
     return np.arange(max(0, count - cap), count) % cap
 
 
-def long_case(backend, dev, n_past, cap, seed, split, nh=8, nkv=4, qscale=0.5):
+def long_case(backend, dev, n_past, cap, seed, split, nh=8, nkv=4, qscale=0.5, device_pos=False):
     hd = 256
     rng = np.random.default_rng(3700 + seed)
     kvd = nkv * hd
@@ -44,7 +46,8 @@ def long_case(backend, dev, n_past, cap, seed, split, nh=8, nkv=4, qscale=0.5):
     out = backend.HipBuffer.alloc(dev, nh * hd)
     pk = backend.HipBuffer.alloc(dev, dev.q8_0_pack_bytes(nh * hd), np.uint8)
     fn = dev.attention_causal_split if split else dev.attention_causal
-    fn(qb, kb, vb, out, n_past, nh, nkv, hd, 1.0 / 16.0, cap, pack=pk)
+    pos = backend.HipBuffer.from_host(dev, np.array([n_past], np.int32)) if device_pos else None
+    fn(qb, kb, vb, out, 0 if device_pos else n_past, nh, nkv, hd, 1.0 / 16.0, cap, pack=pk, d_pos=pos)
     dev.sync()
     got, pack = out.numpy(), pk.numpy()
     for b in (qb, kb, vb, out, pk):
@@ -69,12 +72,13 @@ def attention_f64(q, kr, vr, nh, nkv, hd, scale):
     return out
 
 
-# (n_past, capacity): the LDS form's last capacity, the long form at windows
-# in registers (<= 2048), in one chunk, across the chunk boundary (8191
-# terms a chunk) and over whole chunks, ring windows of a non-power-of-two
-# capacity, and the largest capacity with a full window
+# (n_past, capacity): the LDS form in caches up to and past 6144 positions, the
+# long form on both sides of whole chunks (8191 terms a chunk, windows of 16382
+# and 24573 positions) and over many, and ring windows of a capacity that is no
+# power of two
 LONG_CASES = [(6143, 6144), (0, 6145), (1500, 8192), (4000, 8192), (8190, 8192), (8191, 8192), (16381, 16384),
-              (16383, 16384), (12000, 7000), (40000, 24577)]
+              (16383, 16384), (12000, 7000), (40000, 24577), (16380, 16384), (16382, 16384), (40000, 24573),
+              (10239, 12288), (10240, 12288)]
 
 
 @pytest.mark.parametrize("n_past,cap", LONG_CASES)
@@ -82,6 +86,18 @@ def test_attention_long_bit_exact(backend, orc, dev, n_past, cap):
     got, pack, q, kr, vr = long_case(backend, dev, n_past, cap, n_past % 97, split=False)
     ref = orc.attention_f16(q, kr, vr, len(kr) // 1024 - 1, 8, 4, 256, 1.0 / 16.0)
     assert_bits(got, ref, f"attention n_past {n_past} capacity {cap}")
+    check_pack(orc, pack, got, "long attention")
+
+
+# A position on the device: the launch is the long form's for the capacity, the
+# window may be anything (its register branch up to 2048 positions, one chunk up
+# to 8191, as a captured token step runs them early in a long context).
+@pytest.mark.parametrize("n_past", [0, 5, 95, 700, 2046, 2047, 2048, 4000, 8189, 8190, 8191, 8192, 12287, 13000])
+def test_attention_long_form_short_windows(backend, orc, dev, n_past):
+    cap = 12288
+    got, pack, q, kr, vr = long_case(backend, dev, n_past, cap, n_past % 91, split=False, device_pos=True)
+    ref = orc.attention_f16(q, kr, vr, len(kr) // 1024 - 1, 8, 4, 256, 1.0 / 16.0)
+    assert_bits(got, ref, f"attention n_past {n_past} on the device")
     check_pack(orc, pack, got, "long attention")
 
 

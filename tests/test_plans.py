@@ -16,6 +16,7 @@ import pytest
 import test_gpu_attention_any as attention_any
 import test_gpu_decode as decode
 import test_gpu_gemm as gemm
+import test_gpu_long_context as long_context
 import test_gpu_prefill_ops as prefill_ops
 
 NATIVE = Path(__file__).resolve().parent / "native"
@@ -187,3 +188,12 @@ def test_fast_prefill_test_has_both_folds(plan):
     layer = decode.FAST_LAYER.values()
     got = gemm_plans(plan, [(rows, cols, 150) for rows, cols, _ in layer])
     assert [not p["few_fast"] for p in got] == [relaxed for _, _, relaxed in layer]
+
+
+def test_long_cases_are_long(plan):
+    """The windows of the long-context tests that are meant for the long softmax, on both sides of its chunks."""
+    windows = [min(n_past + 1, cap) for n_past, cap in long_context.LONG_CASES]
+    long = {w for w, p in zip(windows, plan([f"span {w}" for w in windows])) if p["long"]}
+    assert long >= {10241, 16381, 16382, 16383, 16384, 24573}
+    assert {6144, 8191, 8192, 10240} <= set(windows) - long
+    assert plan(["span 12288"])[0]["long"]  # test_attention_long_form_short_windows
