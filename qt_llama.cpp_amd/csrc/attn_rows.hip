@@ -23,6 +23,7 @@
 //     cache (lane = dim, coalesced), several batches ahead, with no barrier.
 // At 512 rows x 8 heads of 256 dims behind 2048 positions this took the three
 // launches from 593 us (two launches, a workgroup a row and kv head) to 340.
+// Which of the forms below, or of decode.hip's, a call takes: plans.h.
 
 #include <algorithm>
 

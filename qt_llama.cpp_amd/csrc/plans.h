@@ -15,7 +15,9 @@ constexpr int kCUs = 256, kSIMDs = 4 * kCUs, kLdsBytes = 160 << 10;  // MI355X; 
 // ---- decode softmax ------------------------------------------------------------
 // The line lies on the widest window of the launch, not on the cache's
 // capacity, and where the weights take as much LDS as LONG's chunk and flags:
-// up to there the LDS form costs no resident workgroup.  Attention in caches
+// up to there the LDS form costs a batch no resident workgroup.  (A launch of
+// one row has at most 256 workgroups, one a CU, and would have LDS for longer
+// windows.)  Attention in caches
 // of 8192 positions, LONG / LDS form: 5310 positions, 4 heads of 64 dims over
 // Q4_0 rows 65.6 / 41.9 us; 2774, 8 heads of 128 over f16 36.8 / 25.4; a window
 // of 1024, 16 heads of 128 over Q8_0/Q4_0 23.2 / 19.5.
