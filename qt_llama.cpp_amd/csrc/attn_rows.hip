@@ -730,6 +730,16 @@ __global__ __launch_bounds__(kRowsShortHD) void attn_rows_short_kernel(const flo
 
 }  // namespace
 
+int load_attn_rows(mrml_hip_ctx *ctx)
+{
+    if (ctx->rows_loaded) return MRML_HIP_OK;
+    hipFuncAttributes attr;
+    if (hipError_t e = hipFuncGetAttributes(&attr, reinterpret_cast<const void *>(attn_rows_short_kernel)))
+        return hip_fail(ctx, e, "attn_rows_short_kernel");
+    ctx->rows_loaded = true;
+    return MRML_HIP_OK;
+}
+
 int launch_attn_rows_short(mrml_hip_ctx *ctx, const float *scores, const void *v_cache, float *out, int n_past0,
                            int rows, int n_heads, int capacity, int wlimit)
 {

@@ -1689,6 +1689,7 @@ int launch_attn_rows(mrml_hip_ctx *ctx, const float *q, int q_stride, const void
                      float *out, int n_past0, int rows, int n_heads, int n_kv_heads, int head_dim, int k_fmt, int v_fmt,
                      float scale, int capacity, void *scratch, int sliding_window)
 {
+    if (int rc = load_attn_rows(ctx)) return rc;
     float *scores = reinterpret_cast<float *>(scratch);
     const int wlimit = attn_window_limit(capacity, sliding_window);
     const AttnRowsPlan plan = attn_rows_plan(n_past0, rows, n_heads, n_kv_heads, head_dim, k_fmt, v_fmt, capacity, wlimit);

@@ -16,6 +16,7 @@ struct mrml_hip_ctx {
     void *ws = nullptr;     // scratch: activation packs and partial results
     size_t ws_bytes = 0;
     void *noalloc_scratch = nullptr;  // the device's copy of the allocation-free GEMM's scratch
+    bool rows_loaded = false;         // attn_rows.hip's code is on the device (load_attn_rows)
     std::string err;
 };
 
@@ -215,6 +216,10 @@ bool attn_rope_ok(int n_heads, int n_kv_heads);
 int launch_attn_rows(mrml_hip_ctx *ctx, const float *q, int q_stride, const void *k_cache, const void *v_cache,
                      float *out, int n_past0, int rows, int n_heads, int n_kv_heads, int head_dim, int k_fmt, int v_fmt,
                      float scale, int capacity, void *scratch, int sliding_window);
+// Brings attn_rows.hip's code onto the device.  The runtime does that at a
+// unit's first launch, 1.6 ms, which would fall on the first long chunk after
+// short ones (those run decode.hip's kernels).
+int load_attn_rows(mrml_hip_ctx *ctx);
 // Its parts in attn_rows.hip, in the forms of attn_rows_plan (plans.h): scores; softmax and weighted sum.
 int launch_attn_rows_scores(mrml_hip_ctx *ctx, const AttnRowsPlan &plan, const float *q, int q_stride,
                             const void *k_cache, int n_past0, int rows, int n_heads, int n_kv_heads, int head_dim,

@@ -601,6 +601,7 @@ inline int prefill_attn_rows(const mrml_hip_gemma2_config &c)
 int prefill_buffers(mrml_hip_ctx *ctx, mrml_hip_gemma2 *m)
 {
     if (m->pf_arena) return MRML_HIP_OK;
+    if (int rc = load_attn_rows(ctx)) return rc;
     const mrml_hip_gemma2_config &c = m->cfg;
     const size_t M = kPrefillChunk, qd = (size_t)c.n_heads * c.head_dim, kvd = (size_t)c.n_kv_heads * c.head_dim;
     const size_t widest = std::max<size_t>(std::max<size_t>(qd, c.dim), c.ffn_dim);
